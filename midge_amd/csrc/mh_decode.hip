@@ -1636,7 +1636,7 @@ int step_plan_create(const DevLayer *layers, int n_layers, StepPlan **out) {
     MH_TRY(plan_alloc(p, &p->h, sizeof(float) * (size_t)L0.top_k * (size_t)L0.ffn, "decode plan h"));
     if (L0.expert_dt == MH_DT_MXFP4) {
         // down scales (bit 1: the expert-group kernel), gate and up scales
-        // (bit 2: with bit 1, the expert-grouped kernels of batches 2-16)
+        // (bit 2: with bit 1, the expert-grouped kernels without a look at the scales)
         unsigned *bad = nullptr;
         MH_TRY(dev_alloc((void **)&bad, sizeof(unsigned), "decode plan scale scan"));
         MH_HIP(hipMemset(bad, 0, sizeof(unsigned)));

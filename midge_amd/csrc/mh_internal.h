@@ -76,7 +76,7 @@ int async_flag(AsyncFlag id, const char *msg, unsigned **dev);
 //   ATTN_SPLIT  attention as four launches instead of k_attn1
 //   COOP        the one-launch decode step as a cooperative launch
 //   Q8_NO_ROWS  long batched int8 GEMVs on the register-operand kernel
-//   BATCH_GEMV  decode steps of 2-16 tokens on the per-assignment GEMVs
+//   BATCH_GEMV  decode steps of several tokens on the per-assignment GEMVs
 //               instead of the expert-grouped matrix-core kernels
 //   SPLIT_ROUTE a stack decode's layer boundary (combine, norm, router,
 //               top-k) as three launches instead of k_combine_route
@@ -152,12 +152,34 @@ bool step_plan_ok(const StepPlan *p);
 // 1 if every MXFP4 scale of the plan's layers is f16-exact (the expert-
 // grouped matrix-core kernels may run them).
 bool step_plan_few(const StepPlan *p);
-// The expert FFN of a decode step of 2-16 tokens on the f16 matrix cores,
-// each routed expert's weights read once for its tokens (mh_grouped.hip): h
-// from xb, then ye, from the top-k kernel's expert-sorted order.
-// grouped_ok: the layer and token count fit.
+// A layer's assignments by expert: order[r] = assignment a of sorted position
+// r, order[N + r] = its expert (unroutable ones last, -1), and the same in
+// groups of up to kGroupTok assignments of one expert. One allocation of
+// group_tab_ints(N) ints (group_tab()).
+constexpr int kGroupTok = 4;
+struct GroupEnt {
+    int expert, cnt, pad[2];
+    int a[kGroupTok];   // cnt assignments
+};
+struct GroupTab {
+    int32_t *order;   // [2 N]
+    int *head;        // [2] groups, routed assignments
+    GroupEnt *ent;    // [groups]
+};
+inline uint64_t group_tab_ints(uint64_t N) { return 2 * N + 8 + N * (sizeof(GroupEnt) / 4); }
+inline GroupTab group_tab(void *p, uint64_t N) {
+    GroupTab t;
+    t.order = (int32_t *)p;
+    t.head = (int *)(t.order + 2 * N);
+    t.ent = (GroupEnt *)(t.head + 8);
+    return t;
+}
+// The expert FFN of a few tokens per expert on the f16 matrix cores, each
+// routed expert's weights read once per group of its tokens (mh_grouped.hip):
+// h from xb, then ye. grouped_ok: the layer and token count fit. exact: every
+// scale of the layer is known to be zero or a power of two in [2^-23, 2^13].
 bool grouped_ok(const DevLayer &L, int n);
-int launch_grouped(const DevLayer &L, int n, const int32_t *order, const float *xb, float *h, float *ye,
+int launch_grouped(const DevLayer &L, int n, const GroupTab &tab, const float *xb, float *h, float *ye, bool exact,
                    hipStream_t s);
 // Runs layers [first, first + n_layers) of a plan in one launch; sel, w and
 // usage are indexed from layer `first`. With gxb (then one layer, gsel and

@@ -110,21 +110,86 @@ __device__ __forceinline__ void wave_topk_token(const float *rl, const float *__
     }
 }
 
-// Assignments a block can sort (16 tokens of up to kMaxTopK slots).
-constexpr int kMaxOrder = 16 * kMaxTopK;
-
-// Rank of key ki among the N distinct keys in sk (LDS): the keys are read in
-// batches of 16 issued together (a read-compare loop waits for each read).
-__device__ __forceinline__ int key_rank(const int *sk, int N, int ki) {
-    int r = 0;
-    for (int j0 = 0; j0 < N; j0 += 16) {
-        int kv[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) kv[j] = j0 + j < N ? sk[j0 + j] : INT32_MAX;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) r += kv[j] < ki;
+// The table of groups of sel[N] (N >= 1), by one whole block of any number of
+// waves: counts per expert, a scan of them in wave 0 (16 experts a lane at
+// most), then each assignment's place. Assignments of one expert land in any
+// order; nothing a kernel computes per assignment depends on it. `mem` is LDS
+// of kGroupMem ints. Before this the last block of the router ranked
+// every assignment against every other, which grows with N^2.
+__device__ __forceinline__ void build_groups(const int32_t *__restrict__ sel, int N, int E, const GroupTab &tab,
+                                             int *mem) {
+    int *cnt = mem, *base = mem + kMaxExperts, *run = mem + 2 * kMaxExperts, *gbase = mem + 3 * kMaxExperts;
+    int *odd = mem + 4 * kMaxExperts;   // unroutable assignments so far
+    const int t = threadIdx.x, T = blockDim.x;
+    for (int e = t; e < E; e += T) {
+        cnt[e] = 0;
+        run[e] = 0;
     }
-    return r;
+    if (t == 0) odd[0] = 0;
+    __syncthreads();
+    for (int i = t; i < N; i += T) {
+        const int e = sel[i];
+        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    if (t < 64) {
+        const int per = (E + 63) >> 6, e0 = t * per;
+        int c = 0, g = 0;
+        for (int e = e0; e < min(e0 + per, E); ++e) {
+            c += cnt[e];
+            g += (cnt[e] + kGroupTok - 1) / kGroupTok;
+        }
+        int ci = c, gi = g;   // inclusive sums over the lanes
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int cu = __shfl_up(ci, o), gu = __shfl_up(gi, o);
+            if (t >= o) {
+                ci += cu;
+                gi += gu;
+            }
+        }
+        if (t == 63) {
+            tab.head[0] = gi;
+            tab.head[1] = ci;
+            odd[1] = ci;
+        }
+        ci -= c;
+        gi -= g;
+        for (int e = e0; e < min(e0 + per, E); ++e) {
+            base[e] = ci;
+            gbase[e] = gi;
+            ci += cnt[e];
+            gi += (cnt[e] + kGroupTok - 1) / kGroupTok;
+        }
+    }
+    __syncthreads();
+    const int vend = odd[1];
+    for (int i = t; i < N; i += T) {
+        const int e = sel[i];
+        if (e < 0 || e >= E) {
+            const int r = vend + atomicAdd(&odd[0], 1);
+            tab.order[r] = i;
+            tab.order[N + r] = -1;
+            continue;
+        }
+        const int j = atomicAdd(&run[e], 1), r = base[e] + j;
+        tab.order[r] = i;
+        tab.order[N + r] = e;
+        GroupEnt *ge = tab.ent + gbase[e] + j / kGroupTok;
+        ge->a[j % kGroupTok] = i;
+        if (j % kGroupTok == 0) {
+            ge->expert = e;
+            ge->cnt = min(kGroupTok, cnt[e] - j);
+        }
+    }
+}
+constexpr int kGroupMem = 4 * kMaxExperts + 2;   // ints of build_groups' LDS
+
+// The table of groups of assignments routed elsewhere (one block).
+__global__ void __launch_bounds__(1024)
+k_groups(const int32_t *__restrict__ sel, int N, int E, GroupTab tab) {
+    __shared__ int mem[kGroupMem];
+    build_groups(sel, N, E, tab, mem);
 }
 
 // moe = sum_i w[i] y_i[r] over a token's k slots in slot order, each product
@@ -148,35 +213,23 @@ __device__ __forceinline__ float slot_sum(const float *__restrict__ w, const flo
     return moe;
 }
 
-// One wave per token. With `order` (one block holding all n tokens, n k <=
-// kMaxOrder), the block then sorts the assignments by expert id, stably,
-// unroutable slots last: order[r] = assignment a, order[n k + r] = sel[a].
-// The expert kernels walk assignments in that order, so the assignments of
-// one expert run side by side and share its weight lines in the caches.
+// One wave per token. With a table (one block holding all n tokens), the
+// block then writes the table of groups: the expert kernels walk assignments
+// in its order, so the assignments of one expert run side by side and share
+// its weight lines in the caches.
 template <int PER>
 __global__ void __launch_bounds__(1024)
 k_topk(const float *__restrict__ rl, const float *__restrict__ bias, int n, int E, int k, int router_norm,
        int unfilled, int32_t *__restrict__ sel, float *__restrict__ w, uint32_t *__restrict__ usage,
-       int32_t *__restrict__ order) {
+       GroupTab tab) {
     const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (t < n)   // wave-uniform
         wave_topk_token<PER>(rl + (size_t)t * E, bias, E, k, router_norm, unfilled, sel + (size_t)t * k,
                              w + (size_t)t * k, usage);
-    if (order == nullptr) return;   // grid-uniform
-    __shared__ int skey[kMaxOrder];
-    const int N = n * k;
+    if (tab.order == nullptr) return;   // grid-uniform
+    __shared__ int mem[kGroupMem];
     __syncthreads();   // every wave's sel stores are visible to the block
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const int e = sel[i];
-        skey[i] = (e >= 0 && e < E ? e : E) * N + i;   // distinct keys
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const int ki = skey[i];
-        const int r = key_rank(skey, N, ki);
-        order[r] = i;
-        order[N + r] = ki / N < E ? ki / N : -1;
-    }
+    build_groups(sel, n * k, E, tab, mem);
 }
 
 // ------------------------------------------------------- expert FFN
@@ -348,19 +401,24 @@ k_combine_norm(float *__restrict__ x, const float *__restrict__ ye, const float 
     for (int64_t r = threadIdx.x; r < H; r += blockDim.x) xb[(size_t)t * H + r] = xt[r] * inv * nw[r];
 }
 
-// The boundary between two layers of a decode of 2-16 tokens, in one launch:
+// The boundary between two layers of a decode of up to kCRTok tokens, in one
+// launch (the first layer of a decode, or a prefill's router, without ye):
 // the previous layer's combine x += sum_i w_i y_i (as k_combine_norm; none
 // before the first layer), this layer's RMSNorm (xb, as k_rmsnorm), its
 // router logits, and per token the top-k and weights (wave_topk_token, as
-// k_topk); the launch's last token sorts the assignments by expert.
+// k_topk); the launch's last token writes the table of groups.
 //   Block (t, g) forms token t's x and xb itself (the same arithmetic in
 //   every block of the token, bit-identical to the separate kernels) and
 //   computes router rows [kCRRows g, +kCRRows), one per wave, the row's loads
 //   issued first. The token's last block to arrive ranks the token and
 //   writes its x back (every block of the token has read it by then); the
-//   launch's last ranked token writes the order. Counters are left at zero.
+//   launch's last ranked token writes the table. Counters are left at zero.
+//   At 40 tokens of a 128-expert layer it takes 23 us, at 64 tokens 24 us
+//   (norm, router GEMV and top-k apart: 25 and 35 us and two launches more).
+//   kCRTok is the engine's own prompt chunk.
 constexpr int kCRRows = 16;       // router rows per block (one per wave)
 constexpr int kCRMaxH = 3072;     // hidden (3 elements per thread)
+constexpr int kCRTok = 64;        // tokens
 // 16-byte chunks of a router row per lane: a row of kCRMaxH elements (int8:
 // 3, f32: 12; loads past the row would re-read its last chunk)
 template <int DT>
@@ -385,7 +443,7 @@ struct CombineRouteArgs {
     int32_t *sel;          // [n][k] out
     float *w;              // [n][k] out
     uint32_t *usage;       // [E] or null
-    int32_t *order;        // [2 n k] out
+    GroupTab tab;          // out
     unsigned *cnt;         // [n + 1] arrival counters
 };
 
@@ -393,9 +451,10 @@ template <int DT, int PER>
 __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
 #pragma clang fp contract(off)
     __shared__ float part[16];
-    __shared__ __attribute__((aligned(16))) float s_xb[kCRMaxH];
+    __shared__ __attribute__((aligned(16))) int s_mem[kGroupMem];   // xb, then the table's counts
+    static_assert(kGroupMem >= kCRMaxH, "xb fits");
+    float *s_xb = (float *)s_mem;
     __shared__ int s_last;
-    __shared__ int skey[kMaxOrder];
     constexpr int CE = mh_chunk<DT>::E;
     constexpr int kV = kCRMaxH / 1024;
     const int t = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -489,7 +548,7 @@ __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
     if (wave == 0)
         wave_topk_token<PER>(A.rl + (size_t)t * E, A.rb, E, k, A.router_norm, A.unfilled, A.sel + (size_t)t * k,
                              A.w + (size_t)t * k, A.usage);
-    // the launch's last ranked token sorts the assignments (as k_topk)
+    // the launch's last ranked token writes the table of groups
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (tid == 0) {
@@ -505,18 +564,7 @@ __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
     }
     __syncthreads();
     if (!s_last) return;
-    const int N = A.n * k;
-    for (int i = tid; i < N; i += 1024) {
-        const int se = A.sel[i];
-        skey[i] = (se >= 0 && se < E ? se : E) * N + i;   // distinct keys
-    }
-    __syncthreads();
-    for (int i = tid; i < N; i += 1024) {
-        const int ki = skey[i];
-        const int r = key_rank(skey, N, ki);
-        A.order[r] = i;
-        A.order[N + r] = ki / N < E ? ki / N : -1;
-    }
+    build_groups(A.sel, A.n * k, E, A.tab, s_mem);
 }
 
 // zeroes n words (a fill kernel: no memset node in a caller's graph)
@@ -649,11 +697,18 @@ int launch_experts(const DevLayer &L, int A, const int32_t *sel, const int32_t *
     return fail(MH_E_DTYPE, "unknown expert dtype %d", L.expert_dt);
 }
 
-// order: null, or [2 n k] for the expert-sorted assignment order (n <= 16).
+int launch_groups(const int32_t *sel, int N, int E, const GroupTab &tab, hipStream_t s) {
+    MH_LAUNCH("groups", k_groups, dim3(1), dim3(1024), 0, s, sel, N, E, tab);
+    return hip_check(hipGetLastError(), "groups launch");
+}
+
+// tab: null, or the table of groups to write (up to 16 tokens by the top-k's
+// own block, more by a launch after it).
 int launch_topk(const float *rl, const float *bias, int n, int E, int k, int router_norm, int unfilled,
-                int32_t *sel, float *w, uint32_t *usage, int32_t *order, hipStream_t s) {
-    if (order && (n > 16 || n * k > kMaxOrder)) return fail(MH_E_ARG, "topk: %d x %d assignments to order", n, k);
-    const int per_block = order ? n : 4;
+                int32_t *sel, float *w, uint32_t *usage, const GroupTab *tab, hipStream_t s) {
+    const bool own = tab && n <= 16;
+    const GroupTab order = own ? *tab : GroupTab{nullptr, nullptr, nullptr};
+    const int per_block = own ? n : 4;
     const dim3 grid((unsigned)((n + per_block - 1) / per_block)), block(64 * per_block);
     // logits per lane: the smallest instantiation that holds E (E <= kMaxExperts)
     if (E <= 128)
@@ -665,29 +720,31 @@ int launch_topk(const float *rl, const float *bias, int n, int E, int k, int rou
     else
         MH_LAUNCH("topk", k_topk<kMaxExperts / 64>, grid, block, 0, s, rl, bias, n, E, k, router_norm, unfilled, sel,
                   w, usage, order);
-    return hip_check(hipGetLastError(), "topk launch");
+    MH_TRY(hip_check(hipGetLastError(), "topk launch"));
+    return tab && !own ? launch_groups(sel, n * k, E, *tab, s) : MH_OK;
 }
 
-// The layer boundary of a decode of 2-16 tokens in one launch
+// The layer boundary of a decode of up to kCRTok tokens in one launch
 // (k_combine_route): MH_E_UNSUPPORTED (error cleared) for shapes it does not
 // take. ye / wprev null: the first layer (no combine).
 bool combine_route_ok(const DevLayer &L, int n) {
     const int CE = L.router.dt == MH_DT_Q8R ? 16 : 4;
     const int chunks = L.router.dt == MH_DT_Q8R ? cr_chunks<MH_DT_Q8R>() : cr_chunks<MH_DT_F32>();
-    return (L.router.dt == MH_DT_Q8R || L.router.dt == MH_DT_F32) && n >= 1 && n <= 16 &&
-           n * L.top_k <= kMaxOrder && L.hidden <= kCRMaxH && L.hidden % CE == 0 &&
+    return (L.router.dt == MH_DT_Q8R || L.router.dt == MH_DT_F32) && n >= 1 &&
+           n <= kCRTok && L.hidden <= kCRMaxH && L.hidden % CE == 0 &&
            L.hidden / CE <= 64 * chunks && L.n_experts <= kMaxExperts && (uintptr_t)L.router.data % 16 == 0 &&
            (uint64_t)L.n_experts * (uint64_t)L.hidden * (L.router.dt == MH_DT_Q8R ? 1u : 4u) < (1ull << 32);
 }
 
 int launch_combine_route(const DevLayer &L, float *x, const float *ye, const float *wprev, int n, float *xb,
-                         float *rl, int32_t *sel, float *w, uint32_t *usage, int32_t *order, hipStream_t s) {
+                         float *rl, int32_t *sel, float *w, uint32_t *usage, const GroupTab &tab, int unfilled,
+                         hipStream_t s) {
     if (!combine_route_ok(L, n)) return MH_E_UNSUPPORTED;
     void *cp = nullptr;
     bool fresh = false;
-    MH_TRY(scratch(S_CROUTE, sizeof(unsigned) * 17, &cp, &fresh));
+    MH_TRY(scratch(S_CROUTE, sizeof(unsigned) * (kCRTok + 1), &cp, &fresh));
     if (fresh) {
-        MH_LAUNCH("zero_counters", k_zero_u32, dim3(1), dim3(64), 0, s, (uint32_t *)cp, 17);
+        MH_LAUNCH("zero_counters", k_zero_u32, dim3(1), dim3(128), 0, s, (uint32_t *)cp, kCRTok + 1);
         MH_TRY(hip_check(hipGetLastError(), "counter clear"));
     }
     CombineRouteArgs A;
@@ -704,13 +761,13 @@ int launch_combine_route(const DevLayer &L, float *x, const float *ye, const flo
     A.rb = L.router_b;
     A.E = L.n_experts;
     A.router_norm = L.router_norm;
-    A.unfilled = -1;
+    A.unfilled = unfilled;
     A.n = n;
     A.rl = rl;
     A.sel = sel;
     A.w = w;
     A.usage = usage;
-    A.order = order;
+    A.tab = tab;
     A.cnt = (unsigned *)cp;
     const dim3 grid((unsigned)n, (unsigned)((L.n_experts + kCRRows - 1) / kCRRows));
 #define CR_LAUNCH(DT, PER) MH_LAUNCH("combine_route", (k_combine_route<DT, PER>), grid, dim3(1024), 0, s, A)
@@ -732,7 +789,8 @@ struct LayerBufs {
     float *xb, *rl, *h, *ye;
     int32_t *sel;
     float *w;
-    int32_t *order;   // [2 n k] expert-sorted assignments (n <= 16), else null
+    GroupTab tab;     // the assignments by expert (null order: none)
+    const int32_t *order() const { return tab.order; }
 };
 
 int layer_bufs(const DevLayer &L, int n, LayerBufs *b) {
@@ -749,38 +807,43 @@ int layer_bufs(const DevLayer &L, int n, LayerBufs *b) {
     b->sel = (int32_t *)p;
     MH_TRY(scratch(S_W, (uint64_t)n * L.top_k * 4, &p));
     b->w = (float *)p;
-    b->order = nullptr;
-    if (n <= 16) {
-        MH_TRY(scratch(S_ORD, (uint64_t)2 * n * L.top_k * 4, &p));
-        b->order = (int32_t *)p;
-    }
+    b->tab = {};
+    const uint64_t N = (uint64_t)n * L.top_k;
+    if (scratch(S_ORD, group_tab_ints(N) * 4, &p) == MH_OK) b->tab = group_tab(p, N);
+    else clear_error();   // over the memory limit: the kernels that walk sel as it is
     return MH_OK;
 }
 
 // Router (rmsnorm, logits, top-k) for n tokens into b->xb / b->sel / b->w
-// (and the expert-sorted order into `order` when it is not null).
+// (and the table of groups when `tab` is not null).
 // x null: b.xb already holds rmsnorm(x) of this layer (k_combine_norm).
 int run_router(const DevLayer &L, const float *x, int n, int unfilled, const LayerBufs &b, uint32_t *usage,
-               int32_t *order, hipStream_t s) {
+               const GroupTab *tab, hipStream_t s) {
     if (x) MH_TRY(launch_rmsnorm(x, L.mlp_norm, b.xb, L.hidden, L.norm_eps, n, s));
     MH_TRY(launch_gemv(L.router, b.xb, b.rl, n, s));
-    return launch_topk(b.rl, L.router_b, n, L.n_experts, L.top_k, L.router_norm, unfilled, b.sel, b.w, usage, order,
+    return launch_topk(b.rl, L.router_b, n, L.n_experts, L.top_k, L.router_norm, unfilled, b.sel, b.w, usage, tab,
                        s);
 }
 
-// few: the layer's MXFP4 scales are known to be f16-exact (a stack's plan
-// scanned them), so 2-16 tokens take the expert-grouped matrix-core kernels
-// (each routed expert read once for its tokens); the BATCH_GEMV switch, or
-// a layer they cannot run, keeps the per-assignment GEMVs.
-// have_xb: b.xb holds this layer's normed input already; next: the next
-// layer, whose RMSNorm is fused into this layer's combine (or null).
+// Two tokens or more through MXFP4 experts take the expert-grouped matrix-core
+// kernels (each routed expert read once for its tokens); the BATCH_GEMV
+// switch, or a layer they cannot run, keeps the per-assignment GEMVs.
+bool decode_grouped(const DevLayer &L, int n, const LayerBufs &b) {
+    return b.order() && !sw(SW_BATCH_GEMV) && !sw(SW_NO_MFMA) && grouped_ok(L, n);
+}
+
+// exact: the layer's scales are known to be carried by f16 (a stack's plan
+// scanned them). have_xb: b.xb holds this layer's normed input already; next:
+// the next layer, whose RMSNorm is fused into this layer's combine (or null).
 int run_decode_layer(const DevLayer &L, float *x, int n, const LayerBufs &b, uint32_t *usage, hipStream_t s,
-                     bool few = false, bool have_xb = false, const DevLayer *next = nullptr) {
-    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, b.order, s));
-    if (few && b.order && !sw(SW_BATCH_GEMV) && grouped_ok(L, n))
-        MH_TRY(launch_grouped(L, n, b.order, b.xb, b.h, b.ye, s));
+                     bool exact = false, bool have_xb = false, const DevLayer *next = nullptr) {
+    const bool grouped = decode_grouped(L, n, b);
+    const bool tab = b.order() && (grouped || n <= 16);   // the GEMVs' walk by expert: up to 16 tokens, in the top-k
+    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, tab ? &b.tab : nullptr, s));
+    if (grouped)
+        MH_TRY(launch_grouped(L, n, b.tab, b.xb, b.h, b.ye, exact, s));
     else
-        MH_TRY(launch_experts(L, n * L.top_k, b.sel, b.order, b.xb, b.h, b.ye, s));
+        MH_TRY(launch_experts(L, n * L.top_k, b.sel, tab ? b.order() : nullptr, b.xb, b.h, b.ye, s));
     if (next) {
         MH_LAUNCH("combine_norm", k_combine_norm, dim3((unsigned)n), dim3(1024), 0, s, x, b.ye, b.w, L.hidden, L.top_k,
                   next->mlp_norm, next->norm_eps, b.xb);
@@ -800,11 +863,29 @@ int run_decode_layer(const DevLayer &L, float *x, int n, const LayerBufs &b, uin
 // to a few 1e-4 of relative error in its logits).
 constexpr int kMfmaMinPerExpert = 8;
 
+bool prefill_gemm(const DevLayer &L, int n) {
+    return prefill_mfma_ok(L) && (int64_t)n * L.top_k >= (int64_t)kMfmaMinPerExpert * L.n_experts;
+}
+
+// A prefill of fewer tokens per expert takes the expert-grouped f16 kernels
+// from two tokens on, as a decode step of as many does (their terms are f32's
+// own accuracy); the per-assignment GEMVs run the rest: one token, other
+// types and shapes, NO_MFMA.
+bool prefill_grouped(const DevLayer &L, int n, const LayerBufs &b) {
+    return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && b.order() && grouped_ok(L, n);
+}
+
+// have_tab: b.tab holds the groups of sel already.
 int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *sel, const float *w, float *x,
-                     const LayerBufs &b, hipStream_t s) {
-    if (prefill_mfma_ok(L) && (int64_t)n * L.top_k >= (int64_t)kMfmaMinPerExpert * L.n_experts)
+                     const LayerBufs &b, bool have_tab, hipStream_t s) {
+    if (prefill_gemm(L, n)) {
         MH_TRY(run_expert_major_mfma(L, n, xb, sel, b.ye, s));
-    else MH_TRY(launch_experts(L, n * L.top_k, sel, nullptr, xb, b.h, b.ye, s));
+    } else if (prefill_grouped(L, n, b)) {
+        if (!have_tab) MH_TRY(launch_groups(sel, n * L.top_k, L.n_experts, b.tab, s));
+        MH_TRY(launch_grouped(L, n, b.tab, xb, b.h, b.ye, false, s));
+    } else {
+        MH_TRY(launch_experts(L, n * L.top_k, sel, have_tab ? b.order() : nullptr, xb, b.h, b.ye, s));
+    }
     if (L.hidden % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)b.ye % 16 == 0)
         MH_LAUNCH("combine_prefill", k_combine_prefill4, dim3((unsigned)((L.hidden / 4 + 255) / 256), (unsigned)n),
                   dim3(256), 0, s, x, b.ye, sel, w, L.hidden, L.top_k, L.n_experts);
@@ -812,6 +893,21 @@ int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *s
         MH_LAUNCH("combine_prefill", k_combine_prefill, dim3((unsigned)((L.hidden + 255) / 256), (unsigned)n), dim3(256), 0,
                   s, x, b.ye, sel, w, L.hidden, L.top_k, L.n_experts);
     return hip_check(hipGetLastError(), "prefill combine launch");
+}
+
+// The router of a prefill (forward_batch, engine/midge.c:591-599: route_topk
+// per token) and the expert-major block on its choice. Up to kCRTok tokens
+// are routed in one launch, which also leaves the table of groups.
+int run_prefill(const DevLayer &L, float *x, int n, const LayerBufs &b, hipStream_t s) {
+    bool have_tab = false;
+    if (b.order() && !sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n)) {
+        MH_TRY(launch_combine_route(L, x, nullptr, nullptr, n, b.xb, b.rl, b.sel, b.w, nullptr, b.tab, 0, s));
+        have_tab = true;
+    } else {
+        have_tab = prefill_grouped(L, n, b);
+        MH_TRY(run_router(L, x, n, 0, b, nullptr, have_tab ? &b.tab : nullptr, s));
+    }
+    return run_expert_major(L, n, b.xb, b.sel, b.w, x, b, have_tab, s);
 }
 
 int check_tokens(int n, const char *what) {
@@ -1057,7 +1153,7 @@ int mh_expert_major_dev(const mh_moe_layer *Lh, int n, const float *xb, const in
     MH_TRY(resolve_dev(x, (uint64_t)n * L.hidden * 4, "mh_expert_major_dev x"));
     LayerBufs b;
     MH_TRY(layer_bufs(L, n, &b));
-    return run_expert_major(L, n, xb, sel, w, x, b, stream());
+    return run_expert_major(L, n, xb, sel, w, x, b, false, stream());
 }
 
 int mh_moe_prefill_dev(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, float *w) {
@@ -1073,8 +1169,7 @@ int mh_moe_prefill_dev(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, fl
     LayerBufs b;
     MH_TRY(layer_bufs(L, n, &b));
     hipStream_t s = stream();
-    MH_TRY(run_router(L, x, n, 0, b, nullptr, nullptr, s));
-    MH_TRY(run_expert_major(L, n, b.xb, b.sel, b.w, x, b, s));
+    MH_TRY(run_prefill(L, x, n, b, s));
     if (sel) MH_HIP(hipMemcpyAsync(sel, b.sel, (size_t)n * L.top_k * 4, hipMemcpyDeviceToDevice, s));
     if (w) MH_HIP(hipMemcpyAsync(w, b.w, (size_t)n * L.top_k * 4, hipMemcpyDeviceToDevice, s));
     return MH_OK;
@@ -1095,8 +1190,7 @@ int mh_moe_prefill(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, float 
     hipStream_t s = stream();
     const size_t xbytes = (size_t)n * L.hidden * 4, kbytes = (size_t)n * L.top_k * 4;
     MH_HIP(hipMemcpyAsync(dx, x, xbytes, hipMemcpyHostToDevice, s));
-    MH_TRY(run_router(L, (float *)dx, n, 0, b, nullptr, nullptr, s));
-    MH_TRY(run_expert_major(L, n, b.xb, b.sel, b.w, (float *)dx, b, s));
+    MH_TRY(run_prefill(L, (float *)dx, n, b, s));
     MH_HIP(hipMemcpyAsync(x, dx, xbytes, hipMemcpyDeviceToHost, s));
     if (sel) MH_HIP(hipMemcpyAsync(sel, b.sel, kbytes, hipMemcpyDeviceToHost, s));
     if (w) MH_HIP(hipMemcpyAsync(w, b.w, kbytes, hipMemcpyDeviceToHost, s));
@@ -1154,8 +1248,8 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
     }
     LayerBufs b;
     MH_TRY(layer_bufs(L0, batch, &b));
-    const bool few = step_plan_few(st->plan);
-    bool fuse = b.order != nullptr && !sw(SW_SPLIT_ROUTE);
+    const bool exact = step_plan_few(st->plan);
+    bool fuse = b.order() && !sw(SW_SPLIT_ROUTE);
     for (int l = 0; l < nl && fuse; l++) fuse = combine_route_ok(st->layers[(size_t)l], batch);
     if (fuse) {
         // each layer boundary (the previous layer's combine, this layer's
@@ -1166,16 +1260,17 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
         auto lsel = [&](int l) { return sel ? sel + (size_t)l * batch * k : b.sel; };
         auto lw = [&](int l) { return w ? w + (size_t)l * batch * k : b.w; };
         auto luse = [&](int l) { return usage ? usage + (size_t)l * L0.n_experts : nullptr; };
-        MH_TRY(launch_combine_route(L0, x, nullptr, nullptr, batch, b.xb, b.rl, lsel(0), lw(0), luse(0), b.order, s));
+        MH_TRY(launch_combine_route(L0, x, nullptr, nullptr, batch, b.xb, b.rl, lsel(0), lw(0), luse(0), b.tab, -1,
+                                    s));
         for (int l = 0; l < nl; l++) {
             const DevLayer &L = st->layers[(size_t)l];
-            if (few && !sw(SW_BATCH_GEMV) && grouped_ok(L, batch))
-                MH_TRY(launch_grouped(L, batch, b.order, b.xb, b.h, b.ye, s));
+            if (decode_grouped(L, batch, b))
+                MH_TRY(launch_grouped(L, batch, b.tab, b.xb, b.h, b.ye, exact, s));
             else
-                MH_TRY(launch_experts(L, batch * k, lsel(l), b.order, b.xb, b.h, b.ye, s));
+                MH_TRY(launch_experts(L, batch * k, lsel(l), b.order(), b.xb, b.h, b.ye, s));
             if (l + 1 < nl) {
                 MH_TRY(launch_combine_route(st->layers[(size_t)l + 1], x, b.ye, lw(l), batch, b.xb, b.rl, lsel(l + 1),
-                                            lw(l + 1), luse(l + 1), b.order, s));
+                                            lw(l + 1), luse(l + 1), b.tab, -1, s));
             } else {
                 MH_LAUNCH("combine_decode", k_combine_decode, dim3((unsigned)((L.hidden + 255) / 256), (unsigned)batch),
                           dim3(256), 0, s, x, b.ye, lw(l), L.hidden, L.top_k);
@@ -1191,7 +1286,7 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
         // every layer after the first takes its normed input from the
         // previous layer's combine
         MH_TRY(run_decode_layer(st->layers[(size_t)l], x, batch, bl,
-                                usage ? usage + (size_t)l * L0.n_experts : nullptr, s, few, l > 0,
+                                usage ? usage + (size_t)l * L0.n_experts : nullptr, s, exact, l > 0,
                                 l + 1 < nl ? &st->layers[(size_t)l + 1] : nullptr));
     }
     return MH_OK;
@@ -1216,7 +1311,7 @@ int mh_stack_apply_dev(mh_stack *st, int layer, const float *xb, const int32_t *
     }
     LayerBufs b;
     MH_TRY(layer_bufs(L, 1, &b));
-    return run_expert_major(L, 1, xb, sel, w, x, b, s);
+    return run_expert_major(L, 1, xb, sel, w, x, b, false, s);
 }
 
 int mh_stack_destroy(mh_stack *st) {

@@ -1,0 +1,120 @@
+"""The expert-grouped f16 kernels past 16 tokens and in short prefills: against
+the per-assignment GEMVs on the same weights, at the edges of their ranges
+(groups of 4, one-launch routing up to 64 tokens, partly filled units of 8
+tiles) and with scales that f16 terms cannot carry."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2, say
+from midge_amd import DevBuf, synth
+from midge_amd.moe import MoELayer, Stack, expert_major_dev, moe_prefill
+from midge_amd.synth import Keys, MoEShape
+from oracle import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+# A layer's update from inputs held to 2^-22 of each column's largest value and
+# f32 sums in another order: 2e-6 of x per token (as test_gpu_moe's SPLIT_TOL).
+TOL = 2e-6
+MID = MoEShape(hidden=256, ffn=192, n_experts=64, top_k=4)
+WIDE = MoEShape(hidden=1536, ffn=1088, n_experts=32, top_k=2)   # ffn / 4 and hidden / 8 leave partial units
+SMALL = MoEShape(hidden=64, ffn=64, n_experts=130, top_k=16)
+
+
+def make(shape, seed, scales="plain", bias=None):
+    keys = Keys(seed)
+    ex = synth.host_layer_experts(shape, keys, 0).copy()
+    if scales != "plain":
+        # expert 1: every gate scale; expert 2: one down scale of the last row
+        val = {"odd": 1.37, "big": 2.0 ** 14, "tiny": 2.0 ** -24, "zero": 0.0, "subnormal": 2.0 ** -20}[scales]
+        v = np.frombuffer(np.float16(val).tobytes(), np.uint8)
+        lay = shape.layout
+        g0 = lay.offset(0, 1, 0, 1)
+        ex[g0:g0 + 2 * shape.ffn * (shape.hidden // 32)] = np.tile(v, shape.ffn * (shape.hidden // 32))
+        d0 = lay.offset(0, 2, 2, 1) + 2 * (shape.hidden * (shape.ffn // 32) - 1)
+        ex[d0:d0 + 2] = v
+    w, s, b, nw = synth.host_router(shape, keys, 0)
+    if bias is not None:
+        b = bias(b)
+    return keys, (ex, w, s, b, nw), MoELayer.host(shape, ex, w, s, b, nw)
+
+
+@pytest.mark.parametrize("shape,n,scales", [
+    (MID, 2, "plain"), (MID, 64, "plain"), (MID, 65, "plain"), (MID, 127, "plain"), (WIDE, 33, "plain"),
+    (SMALL, 3, "plain"), (SMALL, 64, "plain"),
+    (MID, 60, "odd"), (MID, 60, "big"), (MID, 60, "tiny"), (MID, 60, "zero"), (MID, 60, "subnormal"), (WIDE, 70, "odd"),
+], ids=lambda v: v if isinstance(v, (int, str)) else f"{v.hidden}x{v.ffn}e{v.n_experts}")
+def test_short_prefill(mh, path_switch, shape, n, scales):
+    say(f"short prefill {shape.hidden}x{shape.ffn} E={shape.n_experts} n={n} scales={scales}")
+    keys, arrays, lay = make(shape, 11, scales)
+    X = synth.host_x(shape, keys, n, step=2)
+    xg, selg, wg = moe_prefill(lay, X)
+    path_switch("NO_MFMA")
+    xv, selv, wv = moe_prefill(lay, X)
+    xr, selr, _ = po.moe_prefill(po.layer_struct(shape, *arrays), X)
+    lay.release()
+    assert (selg == selv).all() and (selg == selr).all()
+    assert not np.array_equal(xg, xv)   # the matrix cores ran
+    for t in range(n):
+        assert rel_l2(xg[t], xv[t]) < TOL, t
+    assert rel_l2(xg, xr) < 1e-4
+
+
+@pytest.mark.parametrize("shape,n,unfilled", [(MID, 17, False), (MID, 64, False), (MID, 65, True), (WIDE, 40, False),
+                                              (SMALL, 50, True)],
+                         ids=lambda v: f"{v.hidden}x{v.ffn}e{v.n_experts}" if isinstance(v, MoEShape) else str(v))
+def test_stack_many_tokens(mh, path_switch, shape, n, unfilled):
+    say(f"stack decode {shape.hidden}x{shape.ffn} E={shape.n_experts} n={n} unfilled={unfilled}")
+
+    def bias(b):
+        b = np.full_like(b, -1e31)
+        b[[2, 11]] = 0.0
+        return b
+
+    keys, arrays, lay = make(shape, 12, bias=bias if unfilled else None)
+    X, k = synth.host_x(shape, keys, n, step=1), shape.top_k
+    st = Stack([lay], max_batch=n)
+    out = []
+    for gemv in (False, True):
+        path_switch("BATCH_GEMV", gemv)
+        xd, sd, ud = DevBuf.from_array(X), DevBuf(4 * n * k), DevBuf.from_array(np.zeros(shape.n_experts, np.uint32))
+        st.decode(xd, n, sd, usage=ud)
+        mh.sync()
+        out.append((xd.download(np.float32, X.shape), sd.download(np.int32, (n, k)),
+                    ud.download(np.uint32, (shape.n_experts,))))
+        for d in (xd, sd, ud):
+            d.free()
+    st.destroy()
+    lay.release()
+    (xg, sg, ug), (xv, sv, uv) = out
+    assert (sg == sv).all() and (ug == uv).all()
+    assert (ug == np.bincount(sg[sg >= 0], minlength=shape.n_experts)).all()
+    assert not np.array_equal(xg, xv)
+    for t in range(n):
+        assert rel_l2(xg[t], xv[t]) < TOL, t
+    if unfilled:
+        assert (sg[:, 2:] == -1).all()
+
+
+def test_given_routing_with_unroutable_slots(mh, path_switch):
+    """mh_expert_major_dev takes any selection: slots outside [0, E) add nothing."""
+    shape, n = MID, 40
+    say("expert major, unroutable slots")
+    keys, arrays, lay = make(shape, 13)
+    X = synth.host_x(shape, keys, n, step=4)
+    rng = np.random.default_rng(5)
+    sel = rng.integers(-2, shape.n_experts + 2, (n, shape.top_k)).astype(np.int32)
+    sel[7] = -1
+    w = rng.random((n, shape.top_k)).astype(np.float32)
+    out = []
+    for gemv in (False, True):
+        path_switch("NO_MFMA", gemv)
+        bufs = [DevBuf.from_array(a) for a in (X, sel, w, X)]
+        expert_major_dev(lay, n, *bufs)
+        mh.sync()
+        out.append(bufs[3].download(np.float32, X.shape))
+        for d in bufs:
+            d.free()
+    lay.release()
+    assert np.array_equal(out[0][7], X[7])
+    for t in range(n):
+        assert rel_l2(out[0][t], out[1][t]) < TOL, t
