@@ -1,0 +1,53 @@
+"""The scaled-matrix-core prefill at the edges of its tiles (16 rows and tokens,
+passes of up to 8 token tiles, K steps of 128 columns, blocks of 128 rows)
+against the per-assignment GEMVs on the same weights."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2, say
+from midge_amd import DevBuf, synth
+from midge_amd.moe import MoELayer, expert_major_dev
+from midge_amd.synth import Keys, MoEShape
+
+pytestmark = pytest.mark.gpu
+# Three e2m3 terms leave at most 2^-12 of a 32-block's largest value, as a
+# uniform error 2^-12 / sqrt(3) of it, and that value is ~2.2 rms of a normal
+# block: 3.1e-4 of a product sum, once in gate/up and once in down.
+TOL = 6.2e-4
+COUNTS = [1, 0, 15, 16, 17, 127, 128, 129, 257]   # tokens of each expert
+
+
+@pytest.mark.parametrize("hidden,ffn,plain", [(64, 64, False), (64, 192, True), (192, 320, False), (256, 128, False),
+                                              (3328, 64, False), (128, 4608, False)])
+def test_gemm_edges(mh, path_switch, hidden, ffn, plain):
+    say(f"prefill gemm {hidden}x{ffn} plain={plain}")
+    shape = MoEShape(hidden=hidden, ffn=ffn, n_experts=len(COUNTS), top_k=2, act_plain=int(plain))
+    keys = Keys(21)
+    ex = synth.host_layer_experts(shape, keys, 0)
+    w, s, b, nw = synth.host_router(shape, keys, 0)
+    lay = MoELayer.host(shape, ex, w, s, b, nw)
+    rng = np.random.default_rng(hidden + ffn)
+    flat = np.concatenate([np.repeat(np.arange(len(COUNTS)), COUNTS), [-1, len(COUNTS)]]).astype(np.int32)
+    sel = rng.permutation(flat).reshape(-1, 2)   # a token may hold one expert twice: two assignments
+    n = len(sel)
+    wt = rng.uniform(0.5, 1.0, (n, 2)).astype(np.float32)
+    xb = rng.standard_normal((n, hidden)).astype(np.float32)
+    xb[3] = 0.0
+    out = []
+    for gemv in (False, True):
+        path_switch("NO_MFMA", gemv)
+        bufs = [DevBuf.from_array(a) for a in (xb, sel, wt, np.zeros_like(xb))]
+        expert_major_dev(lay, n, *bufs)
+        mh.sync()
+        out.append(bufs[3].download(np.float32, xb.shape))
+        for d in bufs:
+            d.free()
+    lay.release()
+    got, want = out
+    assert not np.array_equal(got, want)   # the matrix cores ran
+    for t in range(n):
+        routed = (sel[t] >= 0) & (sel[t] < len(COUNTS))
+        if not routed.any():
+            assert not got[t].any()
+        else:
+            assert rel_l2(got[t], want[t]) < TOL, (t, sel[t])
