@@ -3,6 +3,9 @@
 //   mh_matvec / mh_matvec_dev   wk_matvec, engine/mkern.h:180-198
 //   mh_row / mh_dequant_dev     wk_row, engine/mkern.h:201-236
 //   mh_rmsnorm_dev              wk_rmsnorm, engine/mkern.h:238-243
+#include <type_traits>
+
+#include "mh_dma.cuh"
 #include "mh_gemv.cuh"
 
 namespace mh {
@@ -89,7 +92,7 @@ k_gemv_rowwave(const uint8_t *__restrict__ W, const void *__restrict__ S, const 
 // ------------------------------------------- batched int8 on the matrix cores
 //
 // Y[b] = diag(S) W X[b] for a batch of columns, reading each weight byte
-// once per 32 columns (the per-column GEMV above reads W once per column).
+// once per 32 or 64 columns (the per-column GEMV above reads W per column).
 // Each column of X is written as a 22-bit fixed-point number under a
 // power-of-two scale, x = 2^sh * (65536 d0 + 256 d1 + d2), with balanced
 // int8 digits d0, d1, d2 (|d0| <= 65). The int8 weights then meet the digits
@@ -99,21 +102,20 @@ k_gemv_rowwave(const uint8_t *__restrict__ W, const void *__restrict__ S, const 
 // error of a dot product ~1e-7, against the f32 sequential sum of mv_q8r,
 // engine/mkern.h:23-31, which rounds at every step).
 
-constexpr int kQ8Cols = 32;            // columns per group: NT 16-column tiles
 constexpr int kQ8MaxK = 65536;         // |A0| <= 127 * 65 * K stays below 2^31
 constexpr int kQ8NonFinite = -100000;  // shift marking a column with inf/nan
 
 typedef int mh_i4 __attribute__((ext_vector_type(4)));
 
-// Digits of column c = 32 * blockIdx.x + blockIdx.y, laid out as the B
+// Digits of column c = 16 * NT * blockIdx.x + blockIdx.y, laid out as the B
 // operand of the MFMA: word (group, kc, digit, n, lane) holds, for lane
-// l = 16 kg + cn, the digits of column 32 group + 16 n + cn at k = 64 kc +
+// l = 16 kg + cn, the digits of column 16 * NT group + 16 n + cn at k = 64 kc +
 // 16 kg .. +15. Columns past `batch` get zero digits.
 template <int NT>
 __global__ void __launch_bounds__(256)
 k_xdigits(const float *__restrict__ X, int K, int batch, uint8_t *__restrict__ xq, int *__restrict__ shift) {
     __shared__ float part[4];
-    const int grp = blockIdx.x, cl = blockIdx.y, c = grp * kQ8Cols + cl;
+    const int grp = blockIdx.x, cl = blockIdx.y, c = grp * 16 * NT + cl;
     const int n = cl >> 4, cn = cl & 15, KC = K >> 6;
     const bool live = c < batch;
     const float *x = X + (size_t)(live ? c : 0) * K;
@@ -288,7 +290,7 @@ k_gemm_q8r(const int8_t *__restrict__ W, const float *__restrict__ S, const uint
         }
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            const int col = grp * kQ8Cols + 16 * n + i;
+            const int col = grp * 16 * NT + 16 * n + i;
             if (col >= batch) continue;
             const int sh = shift[col];
             float *yc = Y + (size_t)col * R;
@@ -321,124 +323,195 @@ k_gemm_q8r(const int8_t *__restrict__ W, const float *__restrict__ S, const uint
     }
 }
 
-// Long int8 matrices (the lm_head) at batch 2+: a wave owns tiles of 16 MT
-// rows, an equal contiguous share of them. Per K super-step of 512 columns
-// it loads two of its rows' next 512 bytes with each 64-lane instruction
-// (contiguous runs of whole rows: the fastest HBM pattern; the matrix-core
-// operand layout, 16 rows x 64 bytes per instruction, streams ~25% slower),
-// writes them to its private LDS buffer at a row stride of 528 bytes (the
-// operand lanes' 16 rows then fall in distinct banks), issues the next
-// super-step's loads, and runs the step's matrix instructions from LDS.
-// Digits as in k_gemm_q8r (L2 hits), DB chunks ahead. 67.6 KB of LDS and
-// under 256 VGPRs: two blocks per CU. (lm_head 201088 x 2880 at batch 32:
-// 252 us with the operand-layout loads; with this kernel and 1024-column
-// super-steps (one block per CU) 226 us at MT = 1, 214 at MT = 2, 208 with
-// the digits four chunks ahead; 200 us with 512-column super-steps.)
-constexpr int kQ8SS = 512;         // bytes of a row per super-step (8 chunks of 64)
-constexpr int kQ8RowLds = 528;     // LDS row stride
-constexpr int kQ8RowWaves = 4;     // waves per block (each with its own buffer)
+// Long int8 matrices (the lm_head) at batch 2+: one block of 8 waves per CU,
+// an equal contiguous share of the 16-row tiles each, in passes of up to 16
+// tiles (wave w: tiles w and w + 8) over all of K. A K step is 128 columns:
+// the block's rows (one load instruction: 128 bytes of each of 8 rows) and
+// the step's digits go straight to LDS, the rows two steps ahead (up to 64 KB
+// of a CU's weights in flight), the digits one (L2 hits, read once per block
+// instead of once per wave). The steps run on across passes: the next pass's
+// first loads fly under this one's last steps. Up to 64 columns meet each
+// weight byte. (lm_head 201088 x 2880 at batch 32: 187 us with each wave
+// reading its digits from L2 and its rows through registers, 144 us this way,
+// 4.2 TB/s in the kernel; the digits had been three times the weights' bytes.)
+// LDS: rows [3][wave][tile][16][8] 16-byte chunks, chunk c of row r at slot
+// c ^ (r % 8) (a read's 8 rows then fall in distinct banks); digits
+// [2][chunk][digit][column tile][64] words as they lie in memory.
+constexpr int kQ8Waves = 8, kQ8MT = 2;
+constexpr int kQ8PassTiles = kQ8Waves * kQ8MT;
+constexpr int kQ8TileLds = 16 * 128, kQ8RowsLds = kQ8PassTiles * kQ8TileLds;
+constexpr int q8_digits_lds(int nt) { return 2 * 3 * nt * 1024; }
+constexpr int q8_lds(int nt) { return 3 * kQ8RowsLds + 2 * q8_digits_lds(nt); }
+static_assert(q8_lds(4) <= 160 * 1024, "LDS per workgroup on gfx950");
 
-template <int NT, int MT, int DB>
-__global__ void __launch_bounds__(64 * kQ8RowWaves, 2)
+template <int NT>
+__global__ void __launch_bounds__(64 * kQ8Waves, 2)
 k_gemm_q8r_rows(const int8_t *__restrict__ W, const float *__restrict__ S, const uint8_t *__restrict__ xq,
                 const int *__restrict__ shift, const float *__restrict__ X, float *__restrict__ Y, int R, int K,
                 int batch) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kQ8RowWaves][16 * MT * kQ8RowLds];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int grp = blockIdx.y, KC = K >> 6, NSS = (K + kQ8SS - 1) / kQ8SS;
+    extern __shared__ __attribute__((aligned(16))) uint8_t qlds[];
+    const uint32_t lds0 = lds_offset(qlds);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = blockIdx.y, KC = K >> 6, ST = (KC + 1) >> 1;   // chunks of 64, steps of two
     const int i = lane & 15, g = lane >> 4;
-    const int64_t T = (R + 16 * MT - 1) / (16 * MT), nw = (int64_t)gridDim.x * kQ8RowWaves, gw = (int64_t)blockIdx.x * kQ8RowWaves + wave;
-    const int tbeg = (int)(gw * T / nw), tend = (int)((gw + 1) * T / nw);
-    uint8_t *buf = lds[wave];
-    const mh_gbytes bp = mh_global(xq + ((size_t)grp * KC * 3 * NT * 64 + lane) * 16);
-    mh_u4 st[8 * MT];    // one super-step of the 16 MT rows: rows 2 j, 2 j + 1 (lane halves), 16 bytes a lane
-    mh_u4 b[DB][3 * NT];
-    auto load_b = [&](int set, int kc) {
-#pragma unroll
-        for (int j = 0; j < 3 * NT; ++j)
-            b[set][j] = *(const mh_u4 __attribute__((address_space(1))) *)(bp + ((size_t)kc * 3 * NT + j) * 1024);
+    const int64_t T = ((int64_t)R + 15) / 16;
+    const int tb = (int)(blockIdx.x * T / gridDim.x), n = (int)((blockIdx.x + 1) * T / gridDim.x) - tb;
+    const int np = (n + kQ8PassTiles - 1) / kQ8PassTiles, total = np * ST;   // n >= 1: the grid is at most T
+    auto pass_beg = [&](int p) { return tb + (int)((int64_t)p * n / np); };
+    // this wave's tiles of a pass: the count (0..2), the first at pass_beg + wave
+    auto pass_tiles = [&](int p) {
+        const int c = pass_beg(p + 1) - pass_beg(p);
+        return c > wave + kQ8Waves ? 2 : c > wave ? 1 : 0;
     };
-    for (int tile = tbeg; tile < tend; ++tile) {
-        const int r0 = tile * 16 * MT;
-        auto load_ss = [&](int ss) {
-            const int o = ss * kQ8SS + 16 * (lane & 31);
+    int sh[NT];
 #pragma unroll
-            for (int j = 0; j < 8 * MT; ++j) {
-                const int r = min(r0 + 2 * j + (lane >> 5), R - 1);
-                st[j] = o < K ? mh_load16(mh_global(W + (size_t)r * K + o)) : mh_u4{0u, 0u, 0u, 0u};
-            }
-        };
-        mh_i4 acc[MT][NT][3];
+    for (int t = 0; t < NT; ++t) {
+        sh[t] = shift[grp * 16 * NT + 16 * t + i];
+        asm volatile("" : "+v"(sh[t]));   // here now: waited for in the steps, it would take their loads with it
+    }
+    const bool vec = R % 4 == 0 && (uintptr_t)Y % 16 == 0;
+
+    // ---- loads: the rows' cursor (pass, step) runs ahead of the math
+    const int swz = (lane & 7) ^ (lane >> 3), cmax = K / 16 - 1;
+    int a_pass = 0, a_st = 0, a_n = 0;
+    const uint8_t *ap[kQ8MT][2] = {};
+    auto issue_a = [&](int buf) __attribute__((always_inline)) -> int {
+        if (a_st == 0) {
+            a_n = pass_tiles(a_pass);
+            const int t0 = pass_beg(a_pass) + wave;
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < kQ8MT; ++m)
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
+                for (int h = 0; h < 2; ++h)
+                    ap[m][h] = (const uint8_t *)W + (size_t)min((t0 + kQ8Waves * m) * 16 + 8 * h + (lane >> 3), R - 1) * K;
+        }
+        const uint32_t o = 16u * (uint32_t)min(8 * a_st + swz, cmax);   // past K: a repeat, not multiplied
+        const uint32_t d = lds0 + (uint32_t)buf * kQ8RowsLds + (uint32_t)wave * (kQ8MT * kQ8TileLds);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) acc[m][n][d] = mh_i4{0, 0, 0, 0};
+        for (int m = 0; m < kQ8MT; ++m) {
+            if (m >= a_n) break;   // wave-uniform
+            dma16(d + m * kQ8TileLds, ap[m][0] + o);
+            dma16(d + m * kQ8TileLds + 1024, ap[m][1] + o);
+        }
+        if (++a_st == ST) {
+            a_st = 0;
+            ++a_pass;
+        }
+        return 2 * a_n;
+    };
+    const uint8_t *bsrc = xq + (size_t)grp * KC * 3 * NT * 1024 + 16 * lane;
+    auto issue_b = [&](int st, int buf) __attribute__((always_inline)) {
+        const uint32_t d = lds0 + 3 * kQ8RowsLds + (uint32_t)buf * q8_digits_lds(NT);
+        const int nw = min(2, KC - 2 * st) * 3 * NT;   // the step's kilobytes of digits
+        for (int j = wave; j < nw; j += kQ8Waves) dma16(d + 1024u * j, bsrc + ((size_t)st * 6 * NT + j) * 1024);
+    };
+
+    mh_i4 acc[kQ8MT][NT][3];
+    auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int d = 0; d + 1 < DB; ++d) load_b(d, min(d, KC - 1));
-        load_ss(0);
-        for (int ss = 0; ss < NSS; ++ss) {
-            // this super-step's rows into LDS (the wave's own LDS accesses
-            // complete in order: the last step's reads are done), then the
-            // next super-step's loads
+        for (int m = 0; m < kQ8MT; ++m)
 #pragma unroll
-            for (int j = 0; j < 8 * MT; ++j)
-                *(mh_u4 *)(buf + (2 * j + (lane >> 5)) * kQ8RowLds + 16 * (lane & 31)) = st[j];
-            if (ss + 1 < NSS) load_ss(ss + 1);
-            const int nc = min(kQ8SS / 64, KC - (kQ8SS / 64) * ss);
-            const uint8_t *ab = buf + i * kQ8RowLds + 16 * g;
-            for (int c = 0; c < nc; c += DB) {
+            for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int h = 0; h < DB; ++h) {
-                    if (c + h >= nc) break;
-                    const int kc = (kQ8SS / 64) * ss + c + h;   // its digits are in set kc % DB = h
-                    load_b((h + DB - 1) % DB, min(kc + DB - 1, KC - 1));
+                for (int d = 0; d < 3; ++d) acc[m][t][d] = mh_i4{0, 0, 0, 0};
+    };
+    auto math = [&](auto mtc, int chunks, const uint8_t *la, const uint8_t *lb) __attribute__((always_inline)) {
+        constexpr int M = decltype(mtc)::value;
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) {
-                        const mh_u4 a = *(const mh_u4 *)(ab + 16 * m * kQ8RowLds + 64 * (c + h));
+        for (int h = 0; h < 2; ++h) {
+            if (h >= chunks) break;   // uniform
+            mh_u4 a[M];
 #pragma unroll
-                        for (int n = 0; n < NT; ++n)
+            for (int m = 0; m < M; ++m)
+                a[m] = *(const mh_u4 *)(la + m * kQ8TileLds + 128 * i + 16 * ((4 * h + g) ^ (i & 7)));
 #pragma unroll
-                            for (int d = 0; d < 3; ++d)
-                                acc[m][n][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                                    (mh_i4)a, (mh_i4)b[h][d * NT + n], acc[m][n][d], 0, 0, 0);
-                    }
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const mh_u4 b = *(const mh_u4 *)(lb + ((h * 3 + d) * NT + t) * 1024 + 16 * lane);
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+                        acc[m][t][d] =
+                            __builtin_amdgcn_mfma_i32_16x16x64_i8((mh_i4)a[m], (mh_i4)b, acc[m][t][d], 0, 0, 0);
                 }
-            }
+        }
+    };
+    auto store = [&](int m, int tile) __attribute__((always_inline)) {
+        const int r0 = tile * 16, row = r0 + 4 * g;
+        float sc[4];   // the rows' scales: a uniform load where the tile is whole (a vector load waits for the loads above)
+        if (r0 + 16 <= R) {
+            const float __attribute__((address_space(4))) *su =
+                (const float __attribute__((address_space(4))) *)(uintptr_t)(S + __builtin_amdgcn_readfirstlane(r0));
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                sc[q] = g < 2 ? (g == 0 ? su[q] : su[4 + q]) : (g == 2 ? su[8 + q] : su[12 + q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sc[q] = S[min(row + q, R - 1)];
         }
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const int col = grp * kQ8Cols + 16 * n + i;
+        for (int t = 0; t < NT; ++t) {
+            const int col = grp * 16 * NT + 16 * t + i;
             if (col >= batch) continue;
-            const int sh = shift[col];
             float *yc = Y + (size_t)col * R;
-            if (sh == kQ8NonFinite) {
+            if (sh[t] == kQ8NonFinite) {
                 // a column holding inf or nan: the plain f32 sum, so the
                 // pattern of infinities and nans is that of mv_q8r
                 const float *xc = X + (size_t)col * K;
 #pragma unroll 1
-                for (int q = 0; q < 4 * MT; ++q) {
-                    const int row = r0 + 16 * (q >> 2) + 4 * g + (q & 3);
-                    if (row >= R) continue;
-                    const int8_t *wr = W + (size_t)row * K;
-                    float t = 0.f;
-                    for (int k = 0; k < K; ++k) t = __builtin_fmaf((float)wr[k], xc[k], t);
-                    yc[row] = t * S[row];
+                for (int q = 0; q < 4; ++q) {
+                    if (row + q >= R) continue;
+                    const int8_t *wr = W + (size_t)(row + q) * K;
+                    float v = 0.f;
+                    for (int k = 0; k < K; ++k) v = __builtin_fmaf((float)wr[k], xc[k], v);
+                    yc[row + q] = v * S[row + q];
                 }
                 continue;
             }
+            float v[4];
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
+            for (int q = 0; q < 4; ++q)
+                v[q] = ldexpf((float)acc[m][t][0][q] * 65536.f + ((float)acc[m][t][1][q] * 256.f + (float)acc[m][t][2][q]),
+                              sh[t]) * sc[q];
+            if (vec && row + 4 <= R) {
+                *(float4 *)(yc + row) = float4{v[0], v[1], v[2], v[3]};
+            } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int row = r0 + 16 * m + 4 * g + q;
-                    if (row >= R) continue;
-                    const float t = (float)acc[m][n][0][q] * 65536.f +
-                                    ((float)acc[m][n][1][q] * 256.f + (float)acc[m][n][2][q]);
-                    yc[row] = ldexpf(t, sh) * S[row];
-                }
+                for (int q = 0; q < 4; ++q)
+                    if (row + q < R) yc[row + q] = v[q];
+            }
         }
+    };
+
+    issue_b(0, 0);
+    (void)issue_a(0);
+    int left = total > 1 ? issue_a(1) : 0;   // loads issued after those of the step at hand
+    int st = 0, pass = 0, mine = pass_tiles(0), ab = 0;
+    clear();
+    for (int it = 0; it < total; ++it) {
+        // step `it` is in LDS, and every wave is past step it - 1, whose
+        // buffers are loaded next
+        if (left == 4) dma_wait<4>();
+        else if (left == 2) dma_wait<2>();
+        else dma_wait<0>();
+        dma_barrier();
+        const int nst = st + 1 == ST ? 0 : st + 1;
+        if (it + 1 < total) issue_b(nst, (it + 1) & 1);
+        left = it + 2 < total ? issue_a(ab == 0 ? 2 : ab - 1) : 0;
+        const uint8_t *la = qlds + ab * kQ8RowsLds + wave * (kQ8MT * kQ8TileLds);
+        const uint8_t *lb = qlds + 3 * kQ8RowsLds + (it & 1) * q8_digits_lds(NT);
+        const int chunks = min(2, KC - 2 * st);
+        if (mine == 2) math(std::integral_constant<int, 2>{}, chunks, la, lb);
+        else if (mine == 1) math(std::integral_constant<int, 1>{}, chunks, la, lb);
+        if (nst == 0) {
+            const int t0 = pass_beg(pass) + wave;
+            if (mine > 0) store(0, t0);
+            if (mine > 1) store(1, t0 + kQ8Waves);
+            clear();
+            if (++pass < np) mine = pass_tiles(pass);
+        }
+        st = nst;
+        ab = ab == 2 ? 0 : ab + 1;
     }
 }
 
@@ -533,43 +606,62 @@ int launch_gemm_q8r(const DevWT &w, const float *x, float *y, int batch, hipStre
         (uintptr_t)w.data % 16 != 0)
         return MH_OK;
     if (sw(SW_NO_MFMA)) return MH_OK;
-    const int groups = (batch + kQ8Cols - 1) / kQ8Cols;
-    const int NT = batch > 16 ? 2 : 1;
-    const uint64_t qbytes = (uint64_t)groups * (K / 64) * 3 * NT * 1024;
-    void *p;
-    MH_TRY(scratch(S_XQ, qbytes + (uint64_t)groups * kQ8Cols * 4, &p));
-    uint8_t *xq = (uint8_t *)p;
-    int *sh = (int *)(xq + qbytes);
-    if (NT == 2)
-        MH_LAUNCH("xdigits", k_xdigits<2>, dim3((unsigned)groups, 32), dim3(256), 0, s, x, (int)K, batch, xq, sh);
-    else
-        MH_LAUNCH("xdigits", k_xdigits<1>, dim3((unsigned)groups, 16), dim3(256), 0, s, x, (int)K, batch, xq, sh);
     // the long tiling when it gives every SIMD two waves, else the K-split one
     const bool longm = (R + Q8Long::rows - 1) / Q8Long::rows * (Q8Long::threads / 64) >= 2 * 4 * device_cus();
-    // long: two blocks per CU, each wave an equal share of the rows
-    const int64_t nlong = std::min<int64_t>((R + Q8Long::rows - 1) / Q8Long::rows, 2 * (int64_t)device_cus());
-    auto go = [&](auto kern, int rows, int threads) {
-        const int64_t nb = longm ? nlong : (R + rows - 1) / rows;
-        MH_LAUNCH("gemm_q8r", kern, dim3((unsigned)nb, (unsigned)groups), dim3(threads), 0, s,
-                  (const int8_t *)w.data, (const float *)w.scales, xq, sh, x, y, (int)R, (int)K, batch);
+    const bool rows = longm && !sw(SW_Q8_NO_ROWS);
+    // groups of up to 64 columns (the row kernel) or 32, as even as 16-column tiles allow
+    const int tiles = (batch + 15) / 16, most = rows ? 4 : 2;
+    const int NT = (tiles + (tiles + most - 1) / most - 1) / ((tiles + most - 1) / most);
+    const int groups = (tiles + NT - 1) / NT;
+    const uint64_t qbytes = (uint64_t)groups * (K / 64) * 3 * NT * 1024;
+    void *p;
+    MH_TRY(scratch(S_XQ, qbytes + (uint64_t)groups * 16 * NT * 4, &p));
+    uint8_t *xq = (uint8_t *)p;
+    int *sh = (int *)(xq + qbytes);
+    auto digits = [&](auto kern) {
+        MH_LAUNCH("xdigits", kern, dim3((unsigned)groups, (unsigned)(16 * NT)), dim3(256), 0, s, x, (int)K, batch, xq, sh);
     };
-    if (longm && !sw(SW_Q8_NO_ROWS)) {
-        // two blocks of 4 waves per CU, each wave 32-row tiles
-        const int64_t nb = std::min<int64_t>((R + 31) / 32 / kQ8RowWaves + 1, 2 * (int64_t)device_cus());
-        auto go2 = [&](auto kern) {
-            MH_LAUNCH("gemm_q8r_rows", kern, dim3((unsigned)nb, (unsigned)groups), dim3(64 * kQ8RowWaves), 0, s,
+    switch (NT) {
+    case 1: digits(k_xdigits<1>); break;
+    case 2: digits(k_xdigits<2>); break;
+    case 3: digits(k_xdigits<3>); break;
+    default: digits(k_xdigits<4>); break;
+    }
+    if (rows) {
+        static uint64_t ready = 0;   // the initialisation whose device has the attributes
+        if (ready != init_epoch()) {
+            const void *f[4] = {(const void *)k_gemm_q8r_rows<1>, (const void *)k_gemm_q8r_rows<2>,
+                                (const void *)k_gemm_q8r_rows<3>, (const void *)k_gemm_q8r_rows<4>};
+            for (int i = 0; i < 4; ++i)
+                MH_HIP(hipFuncSetAttribute(f[i], hipFuncAttributeMaxDynamicSharedMemorySize, q8_lds(i + 1)));
+            ready = init_epoch();
+        }
+        const int64_t nb = std::min<int64_t>((R + 15) / 16, device_cus());
+        auto go = [&](auto kern) {
+            MH_LAUNCH("gemm_q8r_rows", kern, dim3((unsigned)nb, (unsigned)groups), dim3(64 * kQ8Waves), q8_lds(NT), s,
                       (const int8_t *)w.data, (const float *)w.scales, xq, sh, x, y, (int)R, (int)K, batch);
         };
-        // digit chunks in flight: as many as fit beside the staged rows at
-        // two waves per SIMD (three spill at two column groups)
-        if (NT == 2) go2(k_gemm_q8r_rows<2, 2, 2>);
-        else go2(k_gemm_q8r_rows<1, 2, 4>);
-    } else if (longm) {
-        if (NT == 2) go(k_gemm_q8r<2, Q8Long>, Q8Long::rows, Q8Long::threads);
-        else go(k_gemm_q8r<1, Q8Long>, Q8Long::rows, Q8Long::threads);
+        switch (NT) {
+        case 1: go(k_gemm_q8r_rows<1>); break;
+        case 2: go(k_gemm_q8r_rows<2>); break;
+        case 3: go(k_gemm_q8r_rows<3>); break;
+        default: go(k_gemm_q8r_rows<4>); break;
+        }
     } else {
-        if (NT == 2) go(k_gemm_q8r<2, Q8Short>, Q8Short::rows, Q8Short::threads);
-        else go(k_gemm_q8r<1, Q8Short>, Q8Short::rows, Q8Short::threads);
+        // long: two blocks per CU, each wave an equal share of the rows
+        const int64_t nlong = std::min<int64_t>((R + Q8Long::rows - 1) / Q8Long::rows, 2 * (int64_t)device_cus());
+        auto go = [&](auto kern, int krows, int threads) {
+            const int64_t nb = longm ? nlong : (R + krows - 1) / krows;
+            MH_LAUNCH("gemm_q8r", kern, dim3((unsigned)nb, (unsigned)groups), dim3(threads), 0, s,
+                      (const int8_t *)w.data, (const float *)w.scales, xq, sh, x, y, (int)R, (int)K, batch);
+        };
+        if (longm) {
+            if (NT == 2) go(k_gemm_q8r<2, Q8Long>, Q8Long::rows, Q8Long::threads);
+            else go(k_gemm_q8r<1, Q8Long>, Q8Long::rows, Q8Long::threads);
+        } else {
+            if (NT == 2) go(k_gemm_q8r<2, Q8Short>, Q8Short::rows, Q8Short::threads);
+            else go(k_gemm_q8r<1, Q8Short>, Q8Short::rows, Q8Short::threads);
+        }
     }
     *done = true;
     return hip_check(hipGetLastError(), "gemm_q8r launch");

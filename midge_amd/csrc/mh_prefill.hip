@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "mh_dma.cuh"
 #include "mh_internal.h"
 
 namespace mh {
@@ -244,19 +245,11 @@ constexpr int gemm_lds(int nm) { return 2 * kLdsB + 3 * gemm_a(nm) + 3 * kLdsS; 
 static_assert(gemm_lds(2) <= 160 * 1024, "LDS per workgroup on gfx950");
 static_assert(kWaves == kPassTiles, "wave w loads row tile w and token tile w");
 
-// Memory -> LDS without a register in between: lane i's piece lands at
-// lds + 16 i (4 i). The compiler does not see these loads (a builtin makes it
-// wait for all of them at every LDS read): the step's wait below counts them.
-__device__ __forceinline__ void dma16(uint32_t lds, const uint8_t *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
-}
-__device__ __forceinline__ void dma4(uint32_t lds, const uint8_t *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
-}
 // This wave's loads but the last LEFT, and its LDS reads, are done; then all waves.
 template <int LEFT>
 __device__ __forceinline__ void step_wait() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+    dma_wait<LEFT>();
+    dma_barrier();
 }
 
 // MODE 0: gate/up (K = H, rows = F, B rows = tokens through list_tok);
@@ -270,7 +263,7 @@ template <int MODE>
 __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
     constexpr int NM = MODE == 0 ? 2 : 1;   // weight matrices: gate and up, or down
     extern __shared__ __attribute__((aligned(16))) uint8_t glds[];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)glds;
+    const uint32_t lds0 = lds_offset(glds);
     const int K = MODE == 0 ? A.H : A.F;
     const int R = MODE == 0 ? A.F : A.H;
     const int groups = (R + kRows - 1) / kRows;
