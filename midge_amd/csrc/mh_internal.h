@@ -140,8 +140,10 @@ int launch_expert_lists(const int32_t *sel, int N, int E, int k, ExpertLists *ou
 
 // Expert-major prefill with scaled MFMA (mh_prefill.hip): the routed
 // experts of n tokens into ye[n * k][hidden] (slot order); the caller adds
-// them to x with the prefill combine.
+// them to x with the prefill combine. xb null: the records of the normed
+// inputs are in prefill_records already.
 bool prefill_mfma_ok(const DevLayer &L);
+int prefill_records(const DevLayer &L, int n, uint8_t **x, uint8_t **h);
 int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32_t *sel, float *ye,
                           hipStream_t s);
 

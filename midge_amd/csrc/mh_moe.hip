@@ -8,6 +8,7 @@
 //   mh_stack_*                  forward()'s layer loop, MoE half, midge.c:557-560
 #include <vector>
 
+#include "mh_fp6.cuh"
 #include "mh_gemv.cuh"
 
 namespace mh {
@@ -567,6 +568,143 @@ __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
     build_groups(A.sel, A.n * k, E, A.tab, s_mem);
 }
 
+// The router of a prefill of more than kCRTok tokens in one launch: RMSNorm,
+// router logits, top-k and weights of TB tokens per block, and the normed
+// input either as f32 rows (xb) or as the matrix product's records (rec,
+// mh_fp6.cuh), so that it is not written and read again in between.
+//   A lane keeps its 16-element chunks of the tokens' xb in registers and the
+//   waves walk the experts' rows (L2 hits), one row ahead. LDS holds xb with
+//   4 floats after every 32 (a lane's chunks and blocks fall in distinct
+//   banks).
+//   Two tokens share a row's conversions from 1024 tokens on; below that one
+//   token per block keeps more blocks in flight.
+// (norm, one GEMV per token, top-k and the quantizer as four launches took 15
+// + 121 + 6 + 9 us for 2000 tokens of a 32-expert layer and 5 + 33 + 5 + 5 for
+// 512, mostly for reading the router's rows and the norm's output once per
+// token and block; this takes 47 and 14 us.)
+constexpr int kRTThreads = 512;
+constexpr int kRTPad = kCRMaxH / 32 * 36;   // floats of a padded row
+
+struct RouteTokArgs {
+    const float *x;        // [n][H]
+    const float *nw;       // norm weights
+    float eps;
+    int H, E, k, n, router_norm, unfilled;
+    const uint8_t *rw;     // int8 router rows [E][H]
+    const float *rs;       // row scales [E]
+    const float *rb;       // bias [E] or null
+    float *xb;             // [n][H] out, or null
+    uint8_t *rec;          // records out, or null
+    int32_t *sel;          // [n][k] out
+    float *w;              // [n][k] out
+};
+
+template <int PER, int TB>
+__global__ void __launch_bounds__(kRTThreads, TB == 1 ? 4 : 2) k_route_tokens(RouteTokArgs A) {
+#pragma clang fp contract(off)
+    constexpr int kW = kRTThreads / 64, kV = kCRMaxH / kRTThreads;
+    constexpr int CE = mh_chunk<MH_DT_Q8R>::E, kC = cr_chunks<MH_DT_Q8R>();
+    static_assert(CE == 16, "a 32-block holds two chunks");
+    __shared__ float part[kW][TB];
+    __shared__ __attribute__((aligned(16))) float s_xb[TB][kRTPad];
+    __shared__ float s_rl[TB][64 * PER];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int H = A.H, E = A.E, C = H / CE;
+    const int t0 = (int)blockIdx.x * TB, nt = min(TB, A.n - t0);
+    const mh_rsrc rr = gemv_rsrc(A.rw, (uint32_t)E * (uint32_t)H);
+    mh_u4 q[kC];
+    auto load_row = [&](int e) __attribute__((always_inline)) {
+        const uint32_t row = (uint32_t)min(e, E - 1) * (uint32_t)H;
+#pragma unroll
+        for (int j = 0; j < kC; ++j)   // past the row: its last chunk again (xb is zero there)
+            q[j] = __builtin_amdgcn_raw_buffer_load_b128(rr, row + 16u * (uint32_t)min(lane + 64 * j, C - 1), 0, 0);
+    };
+    float v[TB][kV];
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+        const float *xt = A.x + (size_t)min(t0 + b, A.n - 1) * H;
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < kV; ++u) {
+            const int r = tid + kRTThreads * u;
+            v[b][u] = r < H ? xt[r] : 0.f;
+            s = __builtin_fmaf(v[b][u], v[b][u], s);
+        }
+        s = mh_wave_sum(s);
+        if (lane == 0) part[wave][b] = s;
+    }
+    load_row(wave);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < kW; ++i) ss += part[i][b];
+        const float inv = 1.0f / sqrtf(ss / (float)H + A.eps);
+#pragma unroll
+        for (int u = 0; u < kV; ++u) {
+            const int r = tid + kRTThreads * u;
+            if (r < H) {
+                const float xbv = v[b][u] * inv * A.nw[r];
+                s_xb[b][r + (r >> 5) * 4] = xbv;
+                if (A.xb && b < nt) A.xb[(size_t)(t0 + b) * H + r] = xbv;
+            }
+        }
+    }
+    __syncthreads();
+    float xr[TB][kC][CE];
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+        for (int j = 0; j < kC; ++j) {
+            const int c = lane + 64 * j;
+            const float *src = s_xb[b] + min(c, C - 1) * CE + (min(c, C - 1) >> 1) * 4;
+#pragma unroll
+            for (int i = 0; i < CE; i += 4) {
+                const float4 a = *(const float4 *)(src + i);
+                xr[b][j][i] = c < C ? a.x : 0.f;
+                xr[b][j][i + 1] = c < C ? a.y : 0.f;
+                xr[b][j][i + 2] = c < C ? a.z : 0.f;
+                xr[b][j][i + 3] = c < C ? a.w : 0.f;
+            }
+        }
+    for (int e = wave; e < E; e += kW) {
+        mh_u4 cur[kC];
+#pragma unroll
+        for (int j = 0; j < kC; ++j) cur[j] = q[j];
+        load_row(e + kW);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < kC; ++j) acc += mh_dot_chunk<MH_DT_Q8R>(cur[j], xr[b][j]);
+            acc = mh_wave_sum(acc);
+            if (lane == 0) s_rl[b][e] = acc * A.rs[e];
+        }
+    }
+    __syncthreads();
+    if (wave < nt) {
+        const size_t o = (size_t)(t0 + wave) * A.k;
+        wave_topk_token<PER>(s_rl[wave], A.rb, E, A.k, A.router_norm, A.unfilled, A.sel + o, A.w + o, nullptr);
+    } else if (A.rec && wave >= TB) {   // the other waves quantize
+        const int nst = k_steps(H), nb = 4 * nst;
+        for (int u = tid - 64 * TB; u < nt * nb; u += kRTThreads - 64 * TB) {
+            const int b = u / nb, blk = u - b * nb;
+            float vb[32];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float4 a = *(const float4 *)(s_xb[b] + min(blk, H / 32 - 1) * 36 + 4 * j);
+                const bool in = 32 * blk < H;
+                vb[4 * j + 0] = in ? a.x : 0.f;
+                vb[4 * j + 1] = in ? a.y : 0.f;
+                vb[4 * j + 2] = in ? a.z : 0.f;
+                vb[4 * j + 3] = in ? a.w : 0.f;
+            }
+            quant_block(vb, A.rec + ((size_t)(t0 + b) * nst + (blk >> 2)) * kRec, blk & 3);
+        }
+    }
+}
+
 // zeroes n words (a fill kernel: no memset node in a caller's graph)
 __global__ void k_zero_u32(uint32_t *p, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
@@ -784,6 +922,42 @@ int launch_combine_route(const DevLayer &L, float *x, const float *ye, const flo
     return hip_check(hipGetLastError(), "combine/route launch");
 }
 
+// Layers that k_route_tokens takes: an int8 router in whole 16-byte chunks, rows
+// of whole 32-blocks that fit its registers.
+bool route_tokens_ok(const DevLayer &L) {
+    return L.router.dt == MH_DT_Q8R && L.hidden % 32 == 0 && L.hidden <= kCRMaxH && L.n_experts <= kMaxExperts &&
+           (uintptr_t)L.router.data % 16 == 0;
+}
+
+int launch_route_tokens(const DevLayer &L, const float *x, int n, float *xb, uint8_t *rec, int32_t *sel, float *w,
+                        int unfilled, hipStream_t s) {
+    RouteTokArgs A;
+    A.x = x;
+    A.nw = L.mlp_norm;
+    A.eps = L.norm_eps;
+    A.H = (int)L.hidden;
+    A.E = L.n_experts;
+    A.k = L.top_k;
+    A.n = n;
+    A.router_norm = L.router_norm;
+    A.unfilled = unfilled;
+    A.rw = L.router.data;
+    A.rs = (const float *)L.router.scales;
+    A.rb = L.router_b;
+    A.xb = xb;
+    A.rec = rec;
+    A.sel = sel;
+    A.w = w;
+    auto go = [&](auto one, auto two) {
+        if (n < 1024) MH_LAUNCH("route_tokens", one, dim3((unsigned)n), dim3(kRTThreads), 0, s, A);
+        else MH_LAUNCH("route_tokens", two, dim3((unsigned)((n + 1) / 2)), dim3(kRTThreads), 0, s, A);
+    };
+    if (L.n_experts <= 128) go(k_route_tokens<2, 1>, k_route_tokens<2, 2>);
+    else if (L.n_experts <= 256) go(k_route_tokens<4, 1>, k_route_tokens<4, 2>);
+    else go(k_route_tokens<kMaxExperts / 64, 1>, k_route_tokens<kMaxExperts / 64, 2>);
+    return hip_check(hipGetLastError(), "route launch");
+}
+
 // Scratch for a layer call of n tokens.
 struct LayerBufs {
     float *xb, *rl, *h, *ye;
@@ -793,14 +967,18 @@ struct LayerBufs {
     const int32_t *order() const { return tab.order; }
 };
 
-int layer_bufs(const DevLayer &L, int n, LayerBufs *b) {
+// (need_h false: the matrix product's h stays in its records)
+int layer_bufs(const DevLayer &L, int n, LayerBufs *b, bool need_h = true) {
     void *p;
     MH_TRY(scratch(S_XB, (uint64_t)n * L.hidden * 4, &p));
     b->xb = (float *)p;
     MH_TRY(scratch(S_RL, (uint64_t)n * L.n_experts * 4, &p));
     b->rl = (float *)p;
-    MH_TRY(scratch(S_H, (uint64_t)n * L.top_k * L.ffn * 4, &p));
-    b->h = (float *)p;
+    b->h = nullptr;
+    if (need_h) {
+        MH_TRY(scratch(S_H, (uint64_t)n * L.top_k * L.ffn * 4, &p));
+        b->h = (float *)p;
+    }
     MH_TRY(scratch(S_YE, (uint64_t)n * L.top_k * L.hidden * 4, &p));
     b->ye = (float *)p;
     MH_TRY(scratch(S_SEL, (uint64_t)n * L.top_k * 4, &p));
@@ -875,7 +1053,8 @@ bool prefill_grouped(const DevLayer &L, int n, const LayerBufs &b) {
     return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && b.order() && grouped_ok(L, n);
 }
 
-// have_tab: b.tab holds the groups of sel already.
+// have_tab: b.tab holds the groups of sel already; xb null: the records of the
+// normed inputs are written already (prefill_gemm only).
 int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *sel, const float *w, float *x,
                      const LayerBufs &b, bool have_tab, hipStream_t s) {
     if (prefill_gemm(L, n)) {
@@ -897,17 +1076,26 @@ int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *s
 
 // The router of a prefill (forward_batch, engine/midge.c:591-599: route_topk
 // per token) and the expert-major block on its choice. Up to kCRTok tokens
-// are routed in one launch, which also leaves the table of groups.
+// are routed in one launch, which also leaves the table of groups, more in
+// one that also leaves the matrix product's records.
 int run_prefill(const DevLayer &L, float *x, int n, const LayerBufs &b, hipStream_t s) {
     bool have_tab = false;
+    const float *xb = b.xb;
     if (b.order() && !sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n)) {
         MH_TRY(launch_combine_route(L, x, nullptr, nullptr, n, b.xb, b.rl, b.sel, b.w, nullptr, b.tab, 0, s));
         have_tab = true;
+    } else if (n > kCRTok && !sw(SW_SPLIT_ROUTE) && route_tokens_ok(L)) {
+        uint8_t *rec = nullptr, *hq;
+        if (prefill_gemm(L, n)) {
+            MH_TRY(prefill_records(L, n, &rec, &hq));
+            xb = nullptr;
+        }
+        MH_TRY(launch_route_tokens(L, x, n, rec ? nullptr : b.xb, rec, b.sel, b.w, 0, s));
     } else {
         have_tab = prefill_grouped(L, n, b);
         MH_TRY(run_router(L, x, n, 0, b, nullptr, have_tab ? &b.tab : nullptr, s));
     }
-    return run_expert_major(L, n, b.xb, b.sel, b.w, x, b, have_tab, s);
+    return run_expert_major(L, n, xb, b.sel, b.w, x, b, have_tab, s);
 }
 
 int check_tokens(int n, const char *what) {
@@ -1152,7 +1340,7 @@ int mh_expert_major_dev(const mh_moe_layer *Lh, int n, const float *xb, const in
     MH_TRY(resolve_dev(w, (uint64_t)n * L.top_k * 4, "mh_expert_major_dev w"));
     MH_TRY(resolve_dev(x, (uint64_t)n * L.hidden * 4, "mh_expert_major_dev x"));
     LayerBufs b;
-    MH_TRY(layer_bufs(L, n, &b));
+    MH_TRY(layer_bufs(L, n, &b, !prefill_gemm(L, n)));
     return run_expert_major(L, n, xb, sel, w, x, b, false, stream());
 }
 
@@ -1167,12 +1355,10 @@ int mh_moe_prefill_dev(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, fl
     if (sel) MH_TRY(resolve_dev(sel, (uint64_t)n * L.top_k * 4, "mh_moe_prefill_dev sel"));
     if (w) MH_TRY(resolve_dev(w, (uint64_t)n * L.top_k * 4, "mh_moe_prefill_dev w"));
     LayerBufs b;
-    MH_TRY(layer_bufs(L, n, &b));
-    hipStream_t s = stream();
-    MH_TRY(run_prefill(L, x, n, b, s));
-    if (sel) MH_HIP(hipMemcpyAsync(sel, b.sel, (size_t)n * L.top_k * 4, hipMemcpyDeviceToDevice, s));
-    if (w) MH_HIP(hipMemcpyAsync(w, b.w, (size_t)n * L.top_k * 4, hipMemcpyDeviceToDevice, s));
-    return MH_OK;
+    MH_TRY(layer_bufs(L, n, &b, !prefill_gemm(L, n)));
+    if (sel) b.sel = sel;   // written where the caller wants them: a copy each costs a launch
+    if (w) b.w = w;
+    return run_prefill(L, x, n, b, stream());
 }
 
 int mh_moe_prefill(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, float *w) {
@@ -1186,7 +1372,7 @@ int mh_moe_prefill(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, float 
     void *dx;
     MH_TRY(scratch(S_X, (uint64_t)n * L.hidden * 4, &dx));
     LayerBufs b;
-    MH_TRY(layer_bufs(L, n, &b));
+    MH_TRY(layer_bufs(L, n, &b, !prefill_gemm(L, n)));
     hipStream_t s = stream();
     const size_t xbytes = (size_t)n * L.hidden * 4, kbytes = (size_t)n * L.top_k * 4;
     MH_HIP(hipMemcpyAsync(dx, x, xbytes, hipMemcpyHostToDevice, s));

@@ -17,8 +17,9 @@
 //              verbatim (e2m1 nibbles) with e8m0 scales taken exactly from
 //              the f16 powers of two; B = the pass's quantized tokens;
 //              V_MFMA_SCALE_F32_16X16X128_F8F6F4 accumulates all terms in
-//              f32; epilogue bias + clamped SwiGLU -> h
-//   quantize   h -> kTerms planes, as for x
+//              f32; epilogue bias + clamped SwiGLU -> h, which never leaves
+//              the block: its 128 rows are a K step of the down product, and
+//              the block writes them quantized
 //   down       per (pass, 128 rows) over h; epilogue + bias -> y of the
 //              assignment's slot; the existing prefill combine then adds
 //              w * y to each token in ascending expert order.
@@ -39,13 +40,13 @@
 #include <type_traits>
 
 #include "mh_dma.cuh"
+#include "mh_fp6.cuh"
 #include "mh_internal.h"
 
 namespace mh {
 
 namespace {
 
-constexpr int kTerms = 3;      // fp6 terms per activation
 constexpr int kWaves = 8;      // waves per GEMM block (two per SIMD)
 constexpr int kTile = 16;      // rows and tokens of a matrix instruction
 constexpr int kPassTiles = 8;  // token tiles of a pass
@@ -53,10 +54,7 @@ constexpr int kRows = kTile * kWaves;   // weight rows (of each matrix) per bloc
 constexpr int kRG = 4;         // row tiles (of each matrix) per wave: half the block's
 
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v6i __attribute__((ext_vector_type(6)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v32f __attribute__((ext_vector_type(32)));
 
 // ---------------------------------------------------------------- lists
 
@@ -74,6 +72,7 @@ __host__ inline int64_t pass_max(int64_t N, int64_t E) {
 // Positions within an expert's list follow the atomics' order; every output
 // is per assignment, so the order does not change any result.
 constexpr int kPlistMaxE = 4096;
+constexpr int kPB = 8;
 __global__ void __launch_bounds__(1024)
 k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *offs, int *list_tok, int *slot_of, int *poff,
             int *pexp) {
@@ -82,9 +81,17 @@ k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *offs, int *
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     for (int i = t; i < E; i += 1024) cnt[i] = 0;
     __syncthreads();
-    for (int a = t; a < N; a += 1024) {
-        const int e = sel[a];
-        rank[a] = (e >= 0 && e < E) ? atomicAdd(&cnt[e], 1) : -1;
+    // (kPB assignments per thread at a time: their loads are in flight
+    // together, and a list of one batch keeps its ranks in registers)
+    int es[kPB], rk[kPB];
+    for (int a0 = t; a0 < N; a0 += 1024 * kPB) {
+#pragma unroll
+        for (int u = 0; u < kPB; ++u) es[u] = a0 + 1024 * u < N ? sel[a0 + 1024 * u] : -1;
+#pragma unroll
+        for (int u = 0; u < kPB; ++u) {
+            rk[u] = es[u] >= 0 && es[u] < E ? atomicAdd(&cnt[es[u]], 1) : -1;
+            if (N > 1024 * kPB && a0 + 1024 * u < N) rank[a0 + 1024 * u] = rk[u];
+        }
     }
     __syncthreads();
     // thread t owns counters [t * ch, t * ch + ch): local sums (tokens in the
@@ -123,39 +130,27 @@ k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *offs, int *
         poff[E] = (int)(total >> 32);
     }
     __syncthreads();
-    for (int a = t; a < N; a += 1024) {
-        const int r = rank[a];
-        if (r >= 0) {
-            const int p = cnt[sel[a]] + r;
-            list_tok[p] = a / k;
-            slot_of[p] = a;
+    for (int a0 = t; a0 < N; a0 += 1024 * kPB) {
+        if (N > 1024 * kPB) {
+#pragma unroll
+            for (int u = 0; u < kPB; ++u) {
+                es[u] = a0 + 1024 * u < N ? sel[a0 + 1024 * u] : -1;
+                rk[u] = a0 + 1024 * u < N ? rank[a0 + 1024 * u] : -1;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kPB; ++u) {
+            if (rk[u] < 0) continue;
+            const int p = cnt[es[u]] + rk[u];
+            list_tok[p] = (a0 + 1024 * u) / k;
+            slot_of[p] = a0 + 1024 * u;
         }
     }
 }
 
 // ---------------------------------------------------------------- quantize
 
-// A quantized row is a record of kRec bytes per K step of 128 columns (4
-// blocks): the terms' 16-byte low pieces of the 4 blocks (codes 0..20 and a
-// third of code 21), term by term, then the terms' 8-byte high pieces, then
-// per block its terms' e8m0 scales in the bytes of one word. The GEMM takes
-// a step's record with 16-byte loads of whole pieces.
-constexpr int kRecHi = kTerms * 64, kRecSc = kTerms * 96, kRec = 320;
-static_assert(kRecSc + 16 <= kRec && kRec % 16 == 0 && kTerms <= 4, "record layout");
-__host__ __device__ inline int k_steps(int K) { return (K + 127) / 128; }
-
-// e such that m * 2^-e <= 7.5 (the largest e2m3 value), as small as possible.
-__device__ __forceinline__ int fp6_block_exp(float m) {
-    int km;
-    const float fm = frexpf(m, &km);   // m = fm * 2^km, fm in [0.5, 1)
-    return fm <= 0.9375f ? km - 3 : km - 2;
-}
-
-// Rows of K f32 -> records (thread = (row, block)). Each term is the previous
-// residual divided by 2^e and rounded by the hardware converter, which
-// interleaves its two 16-value inputs (even columns, odd columns); its values
-// come back exactly from the inverse converter, so the residuals are exact.
-// A zero block, and a block past K of the last step, keeps e = 0.
+// Rows of K f32 -> records (thread = (row, block); blocks past K are zeros).
 __global__ void __launch_bounds__(256)
 k_quant_terms(const float *__restrict__ in, int rows, int K, uint8_t *__restrict__ q) {
     const int nst = k_steps(K), nb = 4 * nst;
@@ -174,31 +169,7 @@ k_quant_terms(const float *__restrict__ in, int rows, int K, uint8_t *__restrict
 #pragma unroll
         for (int j = 0; j < 32; ++j) v[j] = 0.f;
     }
-    uint8_t *rec = q + ((int64_t)r * nst + (b >> 2)) * kRec;
-    const int g = b & 3;
-    uint32_t sc = 0u;
-#pragma unroll
-    for (int t = 0; t < kTerms; ++t) {
-        float m = 0.f;
-#pragma unroll
-        for (int j = 0; j < 32; ++j) m = fmaxf(m, fabsf(v[j]));
-        const int e = m > 0.f ? max(-126, min(127, fp6_block_exp(m))) : 0;
-        const float scl = ldexpf(1.0f, e);
-        v16f ev, od;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            ev[j] = v[2 * j];
-            od[j] = v[2 * j + 1];
-        }
-        const v6i w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scl);
-        const v32f back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(w, scl);
-#pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] -= back[j];
-        *(uint4 *)(rec + 64 * t + 16 * g) = make_uint4((uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2], (uint32_t)w[3]);
-        *(uint2 *)(rec + kRecHi + 32 * t + 8 * g) = make_uint2((uint32_t)w[4], (uint32_t)w[5]);
-        sc |= (uint32_t)(e + 127) << (8 * t);
-    }
-    *(uint32_t *)(rec + kRecSc + 4 * g) = sc;
+    quant_block(v, q + ((int64_t)r * nst + (b >> 2)) * kRec, b & 3);
 }
 
 // ---------------------------------------------------------------- GEMM
@@ -216,7 +187,7 @@ struct GemmArgs {
     const int *list_tok;   // [N]
     const int *slot_of;    // [N]
     const uint8_t *bq;     // records of the B rows
-    float *hbuf;           // [N][F]  (gate/up output, list order)
+    uint8_t *hq;           // records of h, list order (gate/up output)
     float *ye;             // [n * k][H] (down output, slot order)
     unsigned *err;         // set if a weight scale is not a power of two
 };
@@ -243,6 +214,11 @@ constexpr int gemm_a(int nm) { return nm * kWaves * kLdsAT; }
 constexpr int kLdsS = kWaves * kLdsST;
 constexpr int gemm_lds(int nm) { return 2 * kLdsB + 3 * gemm_a(nm) + 3 * kLdsS; }
 static_assert(gemm_lds(2) <= 160 * 1024, "LDS per workgroup on gfx950");
+// gate/up's h, after the steps: floats per block of 32 rows and per token
+// (the readers' 8 lanes, 2 tokens x 4 blocks, fall in distinct banks)
+constexpr int kHBlk = 36, kHTok = 4 * kHBlk;
+static_assert(kPassTiles * kTile * kHTok * 4 <= gemm_lds(2) && kPassTiles * kTile * 4 == 64 * kWaves && kRows == 128,
+              "a block's h: one thread per token and 32 rows, one K step of the down product");
 static_assert(kWaves == kPassTiles, "wave w loads row tile w and token tile w");
 
 // This wave's loads but the last LEFT, and its LDS reads, are done; then all waves.
@@ -398,25 +374,31 @@ __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
         }
         // lane (m, g) holds rows 4 g .. 4 g + 3 of each row tile for token m
         // of its token tiles
+        const int row0 = rgrp * kRows + kRG * rg * kTile + 4 * g;
+        float4 bias[NM][kRG];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int p = p0 + kTile * (tg + 4 * j) + m;
-            if (p >= p1) continue;
-            float *out = MODE == 0 ? A.hbuf + (size_t)(base + p) * A.F : A.ye + (size_t)A.slot_of[base + p] * A.H;
+        for (int r = 0; r < kRG; ++r) {
+            const size_t ro = (size_t)min(row0 + kTile * r, R - 4) * 4;
+            bias[0][r] = *(const float4 *)(ex + A.off[MODE == 0 ? 2 : 8] + ro);
+            if constexpr (MODE == 0) bias[NM - 1][r] = *(const float4 *)(ex + A.off[5] + ro);
+        }
+        if constexpr (MODE == 0) {
+            // h through LDS, [token][block of 32 rows][32 + 4], then thread
+            // (token, block) quantizes; rows past F are zeros
+            step_wait<0>();   // every wave is past the last step
+            float *lh = (float *)glds;
 #pragma unroll
-            for (int r = 0; r < kRG; ++r) {
-                const int row = rgrp * kRows + (kRG * rg + r) * kTile + 4 * g;
-                if (row >= R) continue;   // wave-uniform: R is a multiple of the tile
-                const float4 b0 = *(const float4 *)(ex + A.off[MODE == 0 ? 2 : 8] + (size_t)row * 4);
-                const float bv[4] = {b0.x, b0.y, b0.z, b0.w};
-                float o[4];
-                if constexpr (MODE == 0) {
-                    const float4 b1 = *(const float4 *)(ex + A.off[5] + (size_t)row * 4);
-                    const float uv[4] = {b1.x, b1.y, b1.z, b1.w};
+            for (int j = 0; j < TN; ++j) {
+#pragma unroll
+                for (int r = 0; r < kRG; ++r) {
+                    const int rr = (kRG * rg + r) * kTile + 4 * g;
+                    const float gb[4] = {bias[0][r].x, bias[0][r].y, bias[0][r].z, bias[0][r].w};
+                    const float ub[4] = {bias[NM - 1][r].x, bias[NM - 1][r].y, bias[NM - 1][r].z, bias[NM - 1][r].w};
+                    float o[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float gg = acc[0][r][j][i] + bv[i];
-                        float uu = acc[NM - 1][r][j][i] + uv[i];
+                        float gg = acc[0][r][j][i] + gb[i];
+                        float uu = acc[NM - 1][r][j][i] + ub[i];
                         if (A.act_plain) {
                             o[i] = gg / (1.0f + expf(-gg)) * uu;
                         } else {
@@ -425,12 +407,25 @@ __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
                             if (uu < -A.limit) uu = -A.limit;
                             o[i] = gg / (1.0f + expf(-A.alpha * gg)) * (uu + 1.0f);
                         }
+                        if (row0 + kTile * r >= R) o[i] = 0.f;   // wave-uniform: R is a multiple of the tile
                     }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) o[i] = acc[0][r][j][i] + bv[i];
+                    *(float4 *)(lh + (kTile * (tg + 4 * j) + m) * kHTok + (rr >> 5) * kHBlk + (rr & 31)) =
+                        float4{o[0], o[1], o[2], o[3]};
                 }
-                *(float4 *)(out + row) = float4{o[0], o[1], o[2], o[3]};
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int p = p0 + kTile * (tg + 4 * j) + m;
+                if (p >= p1) continue;
+                float *out = A.ye + (size_t)A.slot_of[base + p] * A.H + row0;
+#pragma unroll
+                for (int r = 0; r < kRG; ++r) {
+                    const v4f c = acc[0][r][j];
+                    const float4 b = bias[0][r];
+                    if (row0 + kTile * r < R)   // wave-uniform
+                        *(float4 *)(out + kTile * r) = float4{c[0] + b.x, c[1] + b.y, c[2] + b.z, c[3] + b.w};
+                }
             }
         }
     };
@@ -439,6 +434,20 @@ __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
     case 0: run(std::integral_constant<int, 0>{}); break;
     case 1: run(std::integral_constant<int, 1>{}); break;
     default: run(std::integral_constant<int, 2>{}); break;
+    }
+    if constexpr (MODE == 0) {
+        __syncthreads();
+        const int tok = threadIdx.x >> 2, blk = threadIdx.x & 3;
+        if (p0 + tok < p1) {
+            const float *src = (const float *)glds + tok * kHTok + blk * kHBlk;
+            float v[32];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float4 a = *(const float4 *)(src + 4 * j);
+                v[4 * j + 0] = a.x; v[4 * j + 1] = a.y; v[4 * j + 2] = a.z; v[4 * j + 3] = a.w;
+            }
+            quant_block(v, A.hq + ((size_t)(base + p0 + tok) * groups + rgrp) * kRec, blk);
+        }
     }
     if (bad) atomicOr(A.err, 1u);
 }
@@ -474,9 +483,20 @@ bool prefill_mfma_ok(const DevLayer &L) {
            L.n_experts <= kPlistMaxE && L.hidden <= kMfmaMaxH && L.ffn <= kMfmaMaxF && (uintptr_t)L.experts % 16 == 0;
 }
 
+// The records of n tokens' x, then of their h (S_Q scratch).
+int prefill_records(const DevLayer &L, int n, uint8_t **x, uint8_t **h) {
+    const size_t qx = (size_t)kRec * n * k_steps((int)L.hidden);
+    void *p;
+    MH_TRY(scratch(S_Q, qx + (size_t)kRec * n * L.top_k * k_steps((int)L.ffn), &p));
+    *x = (uint8_t *)p;
+    *h = *x + qx;
+    return MH_OK;
+}
+
 // Expert-major MoE of n tokens: x[t] += sum over t's slots, in ascending
 // expert order, of w * expert(xb[t]); ye is [n * k][H] scratch read by the
 // prefill combine (launched by the caller), written for routed slots only.
+// xb null: the router has written the records of x (prefill_records).
 int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32_t *sel, float *ye,
                           hipStream_t s) {
     const int k = L.top_k, E = L.n_experts, N = n * k;
@@ -493,13 +513,8 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
                       &scale_err_dev));
     ExpertLists lists;
     MH_TRY(launch_expert_lists(sel, N, E, k, &lists, s));
-    // quantized activations: the larger of x (n rows of H) and h (N rows of F)
-    const size_t qbytes = kRec * std::max((size_t)n * k_steps(H), (size_t)N * k_steps(F));
-    void *pq, *ph;
-    MH_TRY(scratch(S_Q, qbytes, &pq));
-    MH_TRY(scratch(S_H, sizeof(float) * (size_t)N * F, &ph));
-    uint8_t *q = (uint8_t *)pq;
-    float *hbuf = (float *)ph;
+    uint8_t *qx, *qh;
+    MH_TRY(prefill_records(L, n, &qx, &qh));
 
     // ye rows of unroutable slots are not written: the combine skips them
 
@@ -518,25 +533,23 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
     A.pexp = lists.pexp;
     A.list_tok = lists.list_tok;
     A.slot_of = lists.slot_of;
-    A.bq = q;
-    A.hbuf = hbuf;
+    A.bq = qx;
+    A.hq = qh;
     A.ye = ye;
     A.err = scale_err_dev;
 
-    auto quant = [&](const char *name, const float *in, int rows, int K) {
-        const int64_t thr = (int64_t)rows * 4 * k_steps(K);
-        MH_LAUNCH(name, k_quant_terms, dim3((unsigned)((thr + 255) / 256)), dim3(256), 0, s, in, rows, K, q);
-    };
     // a block for every pass that the assignments can make (those without one return)
     auto grid = [&](int R) {
         const int64_t nb = pass_max(N, E) * ((R + kRows - 1) / kRows);
         return dim3((unsigned)((nb + 7) / 8 * 8));
     };
-    // gate/up over the quantized tokens
-    quant("quant_x", xb, n, H);
+    if (xb) {
+        const int64_t thr = (int64_t)n * 4 * k_steps(H);
+        MH_LAUNCH("quant_x", k_quant_terms, dim3((unsigned)((thr + 255) / 256)), dim3(256), 0, s, xb, n, H, qx);
+    }
+    // gate/up over the quantized tokens, then down over the quantized h
     MH_LAUNCH("moe_gu_mfma", k_moe_gemm<0>, grid(F), dim3(64 * kWaves), gemm_lds(2), s, A);
-    // down over the quantized h (list order)
-    quant("quant_h", hbuf, N, F);
+    A.bq = qh;
     MH_LAUNCH("moe_down_mfma", k_moe_gemm<1>, grid(H), dim3(64 * kWaves), gemm_lds(1), s, A);
     return hip_check(hipGetLastError(), "prefill MFMA launches");
 }
