@@ -20,10 +20,30 @@ __device__ __forceinline__ uint32_t lds_offset(const void *p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)p;
 }
 __device__ __forceinline__ void dma16(uint32_t lds, const uint8_t *p) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t lds, const uint8_t *p) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ uint64_t uniform_addr(const uint8_t *p) {
+    const uint64_t a = (uint64_t)p;
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32;
+}
+// (from a scalar base and 32-bit lane offsets: half the address registers. Five
+// wait states before the load: its scalar operands may come from a vector
+// instruction, and the compiler cannot see that it reads them.)
+__device__ __forceinline__ void dma16(uint32_t lds, const uint8_t *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+                 "v"(off), "s"(uniform_addr(base))
+                 : "memory");
+}
+__device__ __forceinline__ void dma4(uint32_t lds, const uint8_t *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+                 "v"(off), "s"(uniform_addr(base))
+                 : "memory");
 }
 template <int LEFT>
 __device__ __forceinline__ void dma_wait() {

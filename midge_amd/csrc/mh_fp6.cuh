@@ -18,9 +18,10 @@ constexpr int kTerms = 3;   // fp6 terms per activation
 // third of code 21), term by term, then the terms' 8-byte high pieces, then
 // per block its terms' e8m0 scales in the bytes of one word. The GEMM takes
 // a step's record with 16-byte loads of whole pieces.
-constexpr int kRecHi = kTerms * 64, kRecSc = kTerms * 96, kRec = 320;
-static_assert(kRecSc + 16 <= kRec && kRec % 16 == 0 && kTerms <= 4, "record layout");
-__host__ __device__ inline int k_steps(int K) { return (K + 127) / 128; }
+constexpr int kRecHi = kTerms * 64, kRecSc = kTerms * 96, kRec = kTerms * 96 + 16;
+static_assert(kRecSc + 16 == kRec && kTerms <= 4, "record layout");
+// (two steps at least, zeros past K: the GEMM's loads run that far ahead)
+__host__ __device__ inline int k_steps(int K) { return K > 128 ? (K + 127) / 128 : 2; }
 
 // e such that m * 2^-e <= 7.5 (the largest e2m3 value), as small as possible.
 __device__ __forceinline__ int fp6_block_exp(float m) {

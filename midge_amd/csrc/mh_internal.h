@@ -130,11 +130,11 @@ int validate_layer(const mh_moe_layer *L);
 int resolve_layer(const mh_moe_layer *L, DevLayer *out);
 
 // Assignments of sel[N] (N = tokens * k) grouped by expert (mh_prefill.hip):
-// offs[E + 1] into the list, the token (assignment / k) and the slot
-// (assignment) of each list position, the passes before each expert
-// (poff[E + 1]) and each pass's expert; in the S_LIST scratch, E <= 4096.
+// the token (assignment / k) and the slot (assignment) of each list position,
+// the passes over the list and their count; in the S_LIST scratch, E <= 4096.
 struct ExpertLists {
-    int *offs, *list_tok, *slot_of, *poff, *pexp;
+    const void *passes;
+    int *npass, *list_tok, *slot_of;
 };
 int launch_expert_lists(const int32_t *sel, int N, int E, int k, ExpertLists *out, hipStream_t s);
 

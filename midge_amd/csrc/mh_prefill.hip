@@ -5,7 +5,7 @@
 //
 //   lists      assignments (token t, slot i) grouped by expert: counts,
 //              offsets, token of each list position, slot of each position,
-//              and the passes (an expert's tokens in runs of up to 128)
+//              and the passes (an expert's tokens in runs of up to 64)
 //   quantize   xb (per token) -> kTerms planes of fp6 e2m3 with an e8m0
 //              scale per 32-element block: x = sum_t q_t * 2^e_t, each term
 //              the rounding residual of the previous one (each shrinks the
@@ -16,7 +16,7 @@
 //   gate/up    per (pass, 128 row pairs): A = the fp4 gate and up rows
 //              verbatim (e2m1 nibbles) with e8m0 scales taken exactly from
 //              the f16 powers of two; B = the pass's quantized tokens;
-//              V_MFMA_SCALE_F32_16X16X128_F8F6F4 accumulates all terms in
+//              V_MFMA_SCALE_F32_32X32X64_F8F6F4 accumulates all terms in
 //              f32; epilogue bias + clamped SwiGLU -> h, which never leaves
 //              the block: its 128 rows are a K step of the down product, and
 //              the block writes them quantized
@@ -24,16 +24,18 @@
 //              assignment's slot; the existing prefill combine then adds
 //              w * y to each token in ascending expert order.
 //
-// Operand layout of the 16x16x128 instruction with fp4 A and fp6 B: lane l
-// holds A row l % 16 and B column l % 16; with g = l / 16, A's 16 bytes (32
-// e2m1 values) and B's 24 bytes (32 e2m3 values, 6 bits each from the lowest
-// bit up) are columns 32 g .. 32 g + 31 of the step, in order, and each
-// lane's scale covers its own 32 columns. So for K step s (columns 128 s ..
-// 128 s + 127) A lane (m, g) takes 16-byte chunk 4 s + g of row m (one MXFP4
-// block and its scale) and B lane (n, g) block 4 s + g of token n with its
-// scale: activations are quantized in natural 32-column blocks, like the
-// weights. Output lane l: column l % 16, rows 4 (l / 16) + i for
-// accumulator i.
+// Operand layout of the 32x32x64 instruction with fp4 A and fp6 B
+// (measured on gfx950 with one-hot operands): lane l holds A row l % 32 and
+// B column l % 32; with g = l / 32, A's 16 bytes (32 e2m1 values) and B's 24
+// bytes (32 e2m3 values, 6 bits each from the lowest bit up) are columns
+// 32 g .. 32 g + 31 of the instruction, in order, and each lane's scale covers
+// its own 32 columns. So for half h of K step s (columns 128 s + 64 h ..) A
+// lane (m, g) takes 16-byte chunk 4 s + 2 h + g of row m (one MXFP4 block and
+// its scale) and B lane (n, g) the same block of token n with its scale:
+// activations are quantized in natural 32-column blocks, like the weights.
+// Output lane l: column l % 32, rows 8 (i / 4) + 4 g + i % 4 for accumulator
+// i. (The 16x16x128 instruction takes tiles of 16 tokens but runs these
+// operands at half the rate: 4.5 against 9.2 PFLOP/s back to back.)
 #include <stdlib.h>
 
 #include <algorithm>
@@ -42,30 +44,37 @@
 #include "mh_dma.cuh"
 #include "mh_fp6.cuh"
 #include "mh_internal.h"
+#include "mh_mfma16.cuh"
 
 namespace mh {
 
 namespace {
 
-constexpr int kWaves = 8;      // waves per GEMM block (two per SIMD)
-constexpr int kTile = 16;      // rows and tokens of a matrix instruction
-constexpr int kPassTiles = 8;  // token tiles of a pass
-constexpr int kRows = kTile * kWaves;   // weight rows (of each matrix) per block
-constexpr int kRG = 4;         // row tiles (of each matrix) per wave: half the block's
+constexpr int kWaves = 4;      // waves per GEMM block (two blocks per CU)
+constexpr int kTile = 32;      // rows and tokens of a matrix instruction
+constexpr int kPassTiles = 2;  // token tiles of a pass
+constexpr int kLoad = 16;      // rows or tokens of a load instruction
+constexpr int kRows = 128;     // weight rows (of each matrix) per block
+constexpr int kRG = 2;         // row tiles (of each matrix) per wave: half the block's
 
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- lists
 
 // An expert's T tokens run in passes of up to kPassTiles token tiles, as
-// even as tiles allow (260 tokens as 6 + 6 + 5 tiles, not 8 + 8 + 1).
+// even as tiles allow.
 __host__ __device__ inline int pass_tiles(int T) { return (T + kTile - 1) / kTile; }
 __host__ __device__ inline int pass_count(int T) { return (pass_tiles(T) + kPassTiles - 1) / kPassTiles; }
 // the most passes that N assignments over E experts can make
 __host__ inline int64_t pass_max(int64_t N, int64_t E) {
     return std::min<int64_t>(E, N) + N / (kTile * kPassTiles);
 }
+
+// A pass's expert, and what its block needs to find the pass among the
+// expert's: the start and length of the expert's list, the passes before it.
+struct Pass {
+    int e, off, T, before;
+};
 
 // The lists in one block (E <= kPlistMaxE): ranks by LDS atomics, an
 // exclusive scan of the counts and of the passes, then the scatter.
@@ -74,8 +83,7 @@ __host__ inline int64_t pass_max(int64_t N, int64_t E) {
 constexpr int kPlistMaxE = 4096;
 constexpr int kPB = 8;
 __global__ void __launch_bounds__(1024)
-k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *offs, int *list_tok, int *slot_of, int *poff,
-            int *pexp) {
+k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *list_tok, int *slot_of, Pass *passes, int *npass) {
     __shared__ int cnt[kPlistMaxE];
     __shared__ unsigned long long wsum[16];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -119,16 +127,11 @@ k_plist_one(const int32_t *sel, int N, int E, int k, int *rank, int *offs, int *
         if (e < E) {
             const int c = cnt[e], np = pass_count(c), p0 = (int)(run >> 32);
             cnt[e] = (int)run;
-            offs[e] = (int)run;
-            poff[e] = p0;
-            for (int p = 0; p < np; ++p) pexp[p0 + p] = e;
+            for (int p = 0; p < np; ++p) passes[p0 + p] = Pass{e, (int)run, c, p0};
             run += (unsigned)c | ((unsigned long long)np << 32);
         }
     }
-    if (t == 0) {
-        offs[E] = (int)total;
-        poff[E] = (int)(total >> 32);
-    }
+    if (t == 0) *npass = (int)(total >> 32);
     __syncthreads();
     for (int a0 = t; a0 < N; a0 += 1024 * kPB) {
         if (N > 1024 * kPB) {
@@ -181,9 +184,8 @@ struct GemmArgs {
     int E, H, F;
     float alpha, limit;
     int act_plain;
-    const int *offs;       // [E + 1]
-    const int *poff;       // [E + 1] passes before expert e
-    const int *pexp;       // expert of each pass
+    const Pass *passes;
+    const int *npass;
     const int *list_tok;   // [N]
     const int *slot_of;    // [N]
     const uint8_t *bq;     // records of the B rows
@@ -199,42 +201,42 @@ __device__ __forceinline__ int e8m0_of_f16(uint32_t h, unsigned &bad) {
     return (int)((f >> 23) & 0xFFu);  // a zero scale (an e8m0 below f16's range) becomes 2^-127
 }
 
-// LDS of a block. A step's weights are a ring of three, its tokens two.
-//   B    [2][token tile][kRec x 16 tokens]: the tile's low pieces per term as
-//        [token][4], its high pieces per term as [token][2], its scale words
-//        as [token][4], and 256 unused bytes. Pieces are swizzled within a
-//        token (low: block g at g ^ (token / 2) % 4, high: half h at
-//        h ^ (token / 4) % 2) so that a read's lanes fall in distinct banks.
-//   A    [3][matrix][row tile][row][4] 16-byte chunks, swizzled like B's low
-//        pieces
-//   AS   [3][row tile][matrix][row][4] f16 scales
-constexpr int kLdsBT = kRec * kTile, kLdsB = kPassTiles * kLdsBT;
-constexpr int kLdsAT = kTile * 64, kLdsST = 256;
-constexpr int gemm_a(int nm) { return nm * kWaves * kLdsAT; }
-constexpr int kLdsS = kWaves * kLdsST;
-constexpr int gemm_lds(int nm) { return 2 * kLdsB + 3 * gemm_a(nm) + 3 * kLdsS; }
-static_assert(gemm_lds(2) <= 160 * 1024, "LDS per workgroup on gfx950");
-// gate/up's h, after the steps: floats per block of 32 rows and per token
-// (the readers' 8 lanes, 2 tokens x 4 blocks, fall in distinct banks)
-constexpr int kHBlk = 36, kHTok = 4 * kHBlk;
-static_assert(kPassTiles * kTile * kHTok * 4 <= gemm_lds(2) && kPassTiles * kTile * 4 == 64 * kWaves && kRows == 128,
-              "a block's h: one thread per token and 32 rows, one K step of the down product");
-static_assert(kWaves == kPassTiles, "wave w loads row tile w and token tile w");
-
-// This wave's loads but the last LEFT, and its LDS reads, are done; then all waves.
-template <int LEFT>
-__device__ __forceinline__ void step_wait() {
-    dma_wait<LEFT>();
-    dma_barrier();
-}
+// LDS of a block: two steps of weights and tokens, four steps of scales.
+//   B    [2][token] records as in memory: 19 16-byte pieces, an odd number, so
+//        that a read's lanes (one piece of 16 tokens) fall in distinct banks
+//   A    [2][matrix][16 rows][row][4] 16-byte chunks, chunk c of a row at
+//        c ^ (row / 4) % 4 for the same reason
+//   AS   [matrix][row][16] f16 scales
+//   I    [32 rows][matrix][row] biases (two of each where there is one matrix)
+constexpr int kLdsBT = kRec * kLoad, kLdsB = kPassTiles * 2 * kLdsBT;
+constexpr int kLdsAT = kLoad * 64;
+constexpr int gemm_a(int nm) { return nm * (kRows / kLoad) * kLdsAT; }
+constexpr int gemm_s(int nm) { return nm * kRows * 32; }
+constexpr int gemm_lds(int nm) { return 2 * (kLdsB + gemm_a(nm)) + gemm_s(nm) + kWaves * 256; }
+static_assert(2 * gemm_lds(2) <= 160 * 1024 && 2 * gemm_lds(1) <= 160 * 1024, "two blocks per CU");
+static_assert(kWaves * kLoad == kPassTiles * kTile && kWaves * 32 == kRows, "wave w loads 32 rows and 16 tokens");
+static_assert(kRows == 128, "a block's rows of h are one K step of the down product");
 
 // MODE 0: gate/up (K = H, rows = F, B rows = tokens through list_tok);
 // MODE 1: down (K = F, rows = H, B rows = list positions).
-// Block = (pass, 128 rows of each matrix). Wave (rg, tg) = (wave % 2, wave /
-// 2) multiplies row tiles 4 rg .. 4 rg + 3 (of each matrix) with token tiles
-// tg and tg + 4: the waves of a SIMD hold token tiles tg and tg + 2. Per K
-// step of 128 columns wave w loads row tile w two steps ahead and token tile
-// w one step ahead, straight into LDS; one barrier a step.
+// Block = (pass, 128 rows of each matrix), two blocks per CU, so that one
+// block's start, end and waits run under the other's products. Wave (rg, tg)
+// = (wave % 2, wave / 2) multiplies row tiles 2 rg, 2 rg + 1 (of each matrix)
+// with token tile tg. Per K step of 128 columns wave w loads rows 32 w ..
+// 32 w + 31 and 16 tokens straight into LDS. A step has two barriers: after
+// the first the step is in LDS and the waves read their operands, after the
+// second all of it is in registers and its buffers take the step after the
+// next, so that two buffers keep up to two steps in flight under the
+// products (weights alone, with one step in flight, took 118 of 194 us).
+// (gpt-oss-20b layer at 512 and 2000 tokens, gate/up + down us: operands
+// through registers, one wave per SIMD 190 + 140 at 512; 8 waves per block,
+// one block per CU, 16x16x128 tiles and a step's scales per load 151 + 117 and
+// 375 + 293; this 156-170 + 91-96 and 362-383 + 212-222. Without products
+// 134 + 80 and 290 + 186, without loads 105 + 61 and 273 + 150: the load path
+// and the steps' LDS reads and barriers bound it, the matrix instructions
+// alone are 93 us of the 2000-token gate/up. Slower: one persistent block
+// per CU with the steps running across units (157 + 90 and 427 + 263), the
+// same with half the waves a phase behind (167 + 112 and 412 + 288).)
 template <int MODE>
 __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
     constexpr int NM = MODE == 0 ? 2 : 1;   // weight matrices: gate and up, or down
@@ -242,232 +244,307 @@ __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
     const uint32_t lds0 = lds_offset(glds);
     const int K = MODE == 0 ? A.H : A.F;
     const int R = MODE == 0 ? A.F : A.H;
-    const int groups = (R + kRows - 1) / kRows;
+    const int groups = MODE == 0 ? k_steps(R) : (R + kRows - 1) / kRows;   // (h in whole K steps of down)
+    const int nsc = K / 32, S = k_steps(K);
     // XCD-aware order: the dispatcher deals blocks to the 8 XCDs round robin
     // (block b to XCD b % 8), so equal consecutive shares of the (expert, row
     // group, pass) list per XCD keep an expert's tokens, and the weights its
     // passes share, in one L2
-    const int total = A.poff[A.E] * groups, share = (total + 7) / 8;
+    const int total = *A.npass * groups, share = (total + 7) / 8;
     const int lin = (int)(blockIdx.x % 8) * share + (int)(blockIdx.x / 8);
     if ((int)(blockIdx.x / 8) >= share || lin >= total) return;   // block-uniform
-    const int e = A.pexp[lin / groups];
-    const int base = A.offs[e], T = A.offs[e + 1] - base;
-    const int np = A.poff[e + 1] - A.poff[e];
-    const int in_e = lin - A.poff[e] * groups, rgrp = in_e / np, pass = in_e - rgrp * np;
-    const int tiles = pass_tiles(T);
-    const int p0 = pass * tiles / np * kTile, p1 = min((pass + 1) * tiles / np * kTile, T);
-    const int nt = (p1 - p0 + kTile - 1) / kTile;
+    const Pass ps = A.passes[lin / groups];
+    const int np = pass_count(ps.T), tiles = pass_tiles(ps.T);
+    const int in_e = lin - ps.before * groups, rgrp = in_e / np, pass = in_e - rgrp * np;
+    const int p0 = pass * tiles / np * kTile;
+    const int base = ps.off + p0, cnt = min((pass + 1) * tiles / np * kTile, ps.T) - p0;   // the pass's list positions
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-    const int m = l & 15, g = l >> 4;
-    const uint8_t *ex = A.experts + (uint64_t)e * A.stride;
-    const int nsc = K / 32, S = k_steps(K);
+    const int m = l & 31, g = l >> 5, m16 = m & 15;
+    const int rg = wave & 1, tg = wave >> 1;
+    const uint8_t *ex = A.experts + (uint64_t)ps.e * A.stride;
 
-    // ---- this lane's sources
-    const int swz = (l & 3) ^ ((l >> 3) & 3);   // block of the step that this lane's low piece or chunk holds
-    const uint8_t *asrc[NM];
-    {
-        const size_t row = (size_t)min(rgrp * kRows + wave * kTile + (l >> 2), R - 1);
+    // ---- loads: 32-bit lane offsets from scalar bases
+    const uint32_t ldsA = lds0 + 2 * kLdsB, ldsS = ldsA + 2 * gemm_a(NM), ldsI = ldsS + gemm_s(NM);
+    const int swz = (l & 3) ^ ((l >> 4) & 3);   // block of the step that this lane's low piece or chunk holds
+    const int row0 = rgrp * kRows + wave * 32;
+    uint32_t aoff[NM][2], soff[NM];
 #pragma unroll
-        for (int mt = 0; mt < NM; ++mt) asrc[mt] = ex + A.off[MODE == 0 ? 3 * mt : 6] + row * (size_t)(K / 2);
+    for (int mt = 0; mt < NM; ++mt) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            aoff[mt][q] = (uint32_t)A.off[MODE == 0 ? 3 * mt : 6] +
+                          (uint32_t)min(row0 + kLoad * q + (l >> 2), R - 1) * (uint32_t)(K / 2) + 16u * swz;
+        soff[mt] = (uint32_t)A.off[MODE == 0 ? 1 + 3 * mt : 7] + 4u * (l & 7);
     }
-    const uint8_t *ssrc;
-    {
-        const size_t row = (size_t)min(rgrp * kRows + wave * kTile + ((l & 31) >> 1), R - 1);
-        ssrc = ex + (MODE == 0 ? (l < 32 ? A.off[1] : A.off[4]) : A.off[7]) + row * (size_t)(2 * nsc);
-    }
-    const uint8_t *bsrc[3];   // low pieces, high pieces of terms 0-1, the rest
-    {
-        const int tok = kTile * wave;
-        auto rec = [&](int n) {
-            const int p = min(p0 + tok + n, p1 - 1);
-            return A.bq + (size_t)(MODE == 0 ? A.list_tok[base + p] : base + p) * ((size_t)S * kRec);
-        };
-        const int n1 = (l & 31) >> 1, h1 = (l & 1) ^ ((n1 >> 2) & 1);
-        bsrc[0] = rec(l >> 2) + 16 * swz;
-        bsrc[1] = rec(n1) + kRecHi + 32 * (l >> 5) + 16 * h1;
-        bsrc[2] = l < 32 ? rec(n1) + kRecHi + 64 + 16 * h1 : rec(l & 15) + kRecSc + 16 * ((l >> 4) & 1);
-    }
-    static_assert(kTerms == 3, "a token tile's pieces: 5 loads of 64");
-    const uint32_t ldsA = lds0 + 2 * kLdsB, ldsS = ldsA + 3 * gemm_a(NM);
+    constexpr int kALoads = 2 * NM, kBLoads = 5;
     auto issue_a = [&](int st, int buf) __attribute__((always_inline)) {
-        const uint32_t c = 16u * (uint32_t)min(4 * st + swz, nsc - 1);   // past K: a repeat (the tokens are zero there)
+        // (past K: what follows the row, in the expert's blob; the tokens are zero there)
 #pragma unroll
         for (int mt = 0; mt < NM; ++mt)
-            dma16(ldsA + (uint32_t)buf * gemm_a(NM) + (uint32_t)(mt * kWaves + wave) * kLdsAT, asrc[mt] + c);
-        dma4(ldsS + (uint32_t)buf * kLdsS + (uint32_t)wave * kLdsST, ssrc + 4u * (uint32_t)min(2 * st + (l & 1), nsc / 2 - 1));
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                dma16(ldsA + (uint32_t)(buf * gemm_a(NM) + (mt * (kRows / kLoad) + 2 * wave + q) * kLdsAT), ex + 64 * st, aoff[mt][q]);
     };
-    constexpr int kALoads = NM + 1;
-    const bool loads_b = wave < nt;
+    // the scales of 4 steps (32 bytes of a row; 8 rows per load instruction:
+    // one step's 8 bytes at a time took as many cache requests as the weights)
+    auto issue_s = [&](int st) __attribute__((always_inline)) {
+        int lr = l >> 3;
+        asm volatile("" : "+v"(lr));   // opaque: else eight rows' offsets stay in registers
+#pragma unroll
+        for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                dma4(ldsS + (uint32_t)((mt * kRows + wave * 32 + 8 * q) * 32), ex + 8 * st,
+                     soff[mt] + (uint32_t)min(row0 + 8 * q + lr, R - 1) * (uint32_t)(2 * nsc));
+    };
+    const bool loads_b = wave * kLoad < cnt;
+    uint32_t boff[kBLoads];   // pieces l, l + 64, .. of the wave's 16 records
+    const uint8_t *bbase = MODE == 0 ? A.bq : A.bq + (size_t)base * ((size_t)S * kRec);
+    constexpr int kPieces = kRec / 16;
+    static_assert(kLoad * kPieces == 64 * kBLoads - 16, "16 tokens' records: 4 loads of 64 pieces and one of 48");
     auto issue_b = [&](int st, int buf) __attribute__((always_inline)) {
         if (!loads_b) return;   // wave-uniform
-        const uint32_t d = lds0 + (uint32_t)buf * kLdsB + (uint32_t)wave * kLdsBT;
-        const uint32_t o = (uint32_t)st * kRec;
+        const uint32_t d = lds0 + (uint32_t)(buf * kLdsB + wave * kLdsBT);
+        const uint8_t *b = bbase + kRec * st;
 #pragma unroll
-        for (int t = 0; t < kTerms; ++t) dma16(d + 1024u * t, bsrc[0] + (o + 64u * t));
-        dma16(d + 1024u * kTerms, bsrc[1] + o);
-        dma16(d + 1024u * (kTerms + 1), bsrc[2] + o);
+        for (int j = 0; j < kBLoads; ++j)
+            if (j + 1 < kBLoads || l < 48) dma16(d + 1024u * j, b, boff[j]);
     };
 
-    const int rg = wave & 1, tg = wave >> 1;
-    const int lo_off = 64 * m + 16 * (g ^ ((m >> 1) & 3));            // this lane's chunk or low piece
-    const int hi_off = 32 * m + 16 * ((g >> 1) ^ ((m >> 2) & 1)) + 8 * (g & 1);
-    unsigned bad = 0;
-
-    auto run = [&](auto ntc) __attribute__((always_inline)) {
-        constexpr int TN = decltype(ntc)::value;   // this wave's token tiles
-        v4f acc[NM][kRG][TN > 0 ? TN : 1];
+    // ---- math: lane (m, g) of the operands and of the outputs' token m
+    int a_off[2];   // this lane's chunk of half h
 #pragma unroll
-        for (int mt = 0; mt < NM; ++mt)
+    for (int h = 0; h < 2; ++h) a_off[h] = 64 * m16 + 16 * ((2 * h + g) ^ ((m16 >> 2) & 3));
+    unsigned bad = 0;
+    v16f acc[NM][kRG];
+#pragma unroll
+    for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+        for (int r = 0; r < kRG; ++r) acc[mt][r] = v16f{};
+    struct Operands {   // a step's: weights, the tokens' low and high pieces and scales
+        mh_u4 a[2][NM][kRG], b[2][kTerms];
+        uint2 h[2][kTerms];
+        int sb[2];
+    };
+    const uint8_t *la0 = glds + 2 * kLdsB + (2 * kRG * rg + (m >> 4)) * kLdsAT;
+    const uint8_t *lb0 = glds + (kTile * tg + m) * kRec;
+    auto read = [&](int buf, Operands &o) __attribute__((always_inline)) {
+        const uint8_t *la = la0 + buf * gemm_a(NM), *lb = lb0 + buf * kLdsB;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            o.sb[h] = *(const int *)(lb + kRecSc + 8 * h + 4 * g);
+#pragma unroll
+            for (int t = 0; t < kTerms; ++t) {
+                o.b[h][t] = *(const mh_u4 *)(lb + 64 * t + 32 * h + 16 * g);
+                o.h[h][t] = *(const uint2 *)(lb + kRecHi + 32 * t + 16 * h + 8 * g);
+            }
 #pragma unroll
             for (int r = 0; r < kRG; ++r)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[mt][r][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        issue_b(0, 0);
-        issue_a(0, 0);
-        if (S > 1) issue_a(1, 1);
-        int ab = 0;   // st % 3
-        for (int st = 0; st < S; ++st) {
-            // step st's loads are done, and every wave is past step st - 1,
-            // whose buffers the next loads overwrite
-            if (st + 1 < S) step_wait<kALoads>();
-            else step_wait<0>();
-            if (st + 1 < S) issue_b(st + 1, (st + 1) & 1);
-            const int ab2 = ab == 0 ? 2 : ab - 1;   // (st + 2) % 3
-            if (st + 2 < S) issue_a(st + 2, ab2);
-            if constexpr (TN > 0) {
-                const uint8_t *la = glds + 2 * kLdsB + ab * gemm_a(NM) + kRG * rg * kLdsAT + lo_off;
-                const uint8_t *ls = glds + 2 * kLdsB + 3 * gemm_a(NM) + ab * kLdsS + kRG * rg * kLdsST + 8 * m + 2 * g;
-                const uint8_t *lb = glds + (st & 1) * kLdsB + tg * kLdsBT;
-                v8i qb[TN][kTerms];
-                int sb[TN];
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const uint8_t *t0 = lb + 4 * j * kLdsBT;
-                    sb[j] = *(const int *)(t0 + kTile * kRecSc + 16 * m + 4 * g);
-#pragma unroll
-                    for (int t = 0; t < kTerms; ++t) {
-                        const mh_u4 lo = *(const mh_u4 *)(t0 + 1024 * t + lo_off);
-                        const uint2 hi = *(const uint2 *)(t0 + 1024 * kTerms + 512 * t + hi_off);
-                        qb[j][t] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, 0, 0};
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < kRG; ++r) {
-#pragma unroll
-                    for (int mt = 0; mt < NM; ++mt) {
-                        const mh_u4 a = *(const mh_u4 *)(la + (mt * kWaves + r) * kLdsAT);
-                        const int sa = e8m0_of_f16(*(const uint16_t *)(ls + r * kLdsST + 128 * mt), bad);
-                        const v8i qa = v8i{(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            v4f c = acc[mt][r][j];
-                            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qa, qb[j][0], c, 4, 2, 0, sa, 0, sb[j]);
-                            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qa, qb[j][1], c, 4, 2, 0, sa, 1, sb[j]);
-                            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qa, qb[j][2], c, 4, 2, 0, sa, 2, sb[j]);
-                            acc[mt][r][j] = c;
-                        }
-                    }
-                }
-            }
-            ab = ab == 2 ? 0 : ab + 1;
-        }
-        // lane (m, g) holds rows 4 g .. 4 g + 3 of each row tile for token m
-        // of its token tiles
-        const int row0 = rgrp * kRows + kRG * rg * kTile + 4 * g;
-        float4 bias[NM][kRG];
-#pragma unroll
-        for (int r = 0; r < kRG; ++r) {
-            const size_t ro = (size_t)min(row0 + kTile * r, R - 4) * 4;
-            bias[0][r] = *(const float4 *)(ex + A.off[MODE == 0 ? 2 : 8] + ro);
-            if constexpr (MODE == 0) bias[NM - 1][r] = *(const float4 *)(ex + A.off[5] + ro);
-        }
-        if constexpr (MODE == 0) {
-            // h through LDS, [token][block of 32 rows][32 + 4], then thread
-            // (token, block) quantizes; rows past F are zeros
-            step_wait<0>();   // every wave is past the last step
-            float *lh = (float *)glds;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-#pragma unroll
-                for (int r = 0; r < kRG; ++r) {
-                    const int rr = (kRG * rg + r) * kTile + 4 * g;
-                    const float gb[4] = {bias[0][r].x, bias[0][r].y, bias[0][r].z, bias[0][r].w};
-                    const float ub[4] = {bias[NM - 1][r].x, bias[NM - 1][r].y, bias[NM - 1][r].z, bias[NM - 1][r].w};
-                    float o[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float gg = acc[0][r][j][i] + gb[i];
-                        float uu = acc[NM - 1][r][j][i] + ub[i];
-                        if (A.act_plain) {
-                            o[i] = gg / (1.0f + expf(-gg)) * uu;
-                        } else {
-                            if (gg > A.limit) gg = A.limit;
-                            if (uu > A.limit) uu = A.limit;
-                            if (uu < -A.limit) uu = -A.limit;
-                            o[i] = gg / (1.0f + expf(-A.alpha * gg)) * (uu + 1.0f);
-                        }
-                        if (row0 + kTile * r >= R) o[i] = 0.f;   // wave-uniform: R is a multiple of the tile
-                    }
-                    *(float4 *)(lh + (kTile * (tg + 4 * j) + m) * kHTok + (rr >> 5) * kHBlk + (rr & 31)) =
-                        float4{o[0], o[1], o[2], o[3]};
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int p = p0 + kTile * (tg + 4 * j) + m;
-                if (p >= p1) continue;
-                float *out = A.ye + (size_t)A.slot_of[base + p] * A.H + row0;
-#pragma unroll
-                for (int r = 0; r < kRG; ++r) {
-                    const v4f c = acc[0][r][j];
-                    const float4 b = bias[0][r];
-                    if (row0 + kTile * r < R)   // wave-uniform
-                        *(float4 *)(out + kTile * r) = float4{c[0] + b.x, c[1] + b.y, c[2] + b.z, c[3] + b.w};
-                }
-            }
+                for (int mt = 0; mt < NM; ++mt)
+                    o.a[h][mt][r] = *(const mh_u4 *)(la + (mt * (kRows / kLoad) + 2 * r) * kLdsAT + a_off[h]);
         }
     };
-    const int tn = nt > tg ? (nt > tg + 4 ? 2 : 1) : 0;   // wave-uniform
-    switch (tn) {
-    case 0: run(std::integral_constant<int, 0>{}); break;
-    case 1: run(std::integral_constant<int, 1>{}); break;
-    default: run(std::integral_constant<int, 2>{}); break;
-    }
-    if constexpr (MODE == 0) {
-        __syncthreads();
-        const int tok = threadIdx.x >> 2, blk = threadIdx.x & 3;
-        if (p0 + tok < p1) {
-            const float *src = (const float *)glds + tok * kHTok + blk * kHBlk;
-            float v[32];
+    // The e8m0 scales of this lane's rows for 4 steps: byte 2 (s % 2) + h of
+    // word s / 2 is block 4 s + 2 h + g's (2^0 past K); two steps later word 1
+    // moves to word 0.
+    uint32_t sw4[NM][kRG][2];
+    auto scales = [&](int st) __attribute__((always_inline)) {
+        const uint8_t *ls = glds + 2 * (kLdsB + gemm_a(NM)) + (kRG * rg * kTile + m) * 32;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 a = *(const float4 *)(src + 4 * j);
-                v[4 * j + 0] = a.x; v[4 * j + 1] = a.y; v[4 * j + 2] = a.z; v[4 * j + 3] = a.w;
+        for (int r = 0; r < kRG; ++r)
+#pragma unroll
+            for (int mt = 0; mt < NM; ++mt) {
+                const uint8_t *p = ls + (mt * kRows + r * kTile) * 32;
+                const mh_u4 v[2] = {*(const mh_u4 *)p, *(const mh_u4 *)(p + 16)};
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    uint32_t x = 0u;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {   // blocks 8 w + 2 i + g
+                        const uint32_t d = dword_of(v[w], i);
+                        const bool in = 4 * st + 8 * w + 2 * i < nsc;   // uniform
+                        unsigned b1 = 0u;
+                        const uint32_t e = (uint32_t)e8m0_of_f16(g ? d >> 16 : d & 0xFFFFu, b1);
+                        bad |= in ? b1 : 0u;
+                        x |= (in ? e : 127u) << (8 * i);
+                    }
+                    sw4[mt][r][w] = x;
+                }
+                __builtin_amdgcn_sched_barrier(0);   // (one row tile's at a time: registers)
             }
-            quant_block(v, A.hq + ((size_t)(base + p0 + tok) * groups + rgrp) * kRec, blk);
+    };
+    auto math = [&](auto bufc, const Operands &o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v8i qa[NM][kRG], qb[kTerms];
+#pragma unroll
+            for (int r = 0; r < kRG; ++r)
+#pragma unroll
+                for (int mt = 0; mt < NM; ++mt) {
+                    const mh_u4 a = o.a[h][mt][r];
+                    qa[mt][r] = v8i{(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
+                }
+#pragma unroll
+            for (int t = 0; t < kTerms; ++t)
+                qb[t] = v8i{(int)o.b[h][t].x, (int)o.b[h][t].y, (int)o.b[h][t].z, (int)o.b[h][t].w,
+                            (int)o.h[h][t].x, (int)o.h[h][t].y, 0, 0};
+            // (term by term: consecutive instructions add into different tiles)
+            auto term = [&](auto hc, auto tc) __attribute__((always_inline)) {
+                constexpr int t = decltype(tc)::value, byte = 2 * decltype(bufc)::value + decltype(hc)::value;
+#pragma unroll
+                for (int r = 0; r < kRG; ++r)
+#pragma unroll
+                    for (int mt = 0; mt < NM; ++mt)
+                        acc[mt][r] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                            qa[mt][r], qb[t], acc[mt][r], 4, 2, byte, (int)sw4[mt][r][0], t, o.sb[h]);
+            };
+            auto terms = [&](auto hc) __attribute__((always_inline)) {
+                term(hc, std::integral_constant<int, 0>{});
+                term(hc, std::integral_constant<int, 1>{});
+                term(hc, std::integral_constant<int, 2>{});
+            };
+            if (h == 0) terms(std::integral_constant<int, 0>{});
+            else terms(std::integral_constant<int, 1>{});
+        }
+    };
+    const bool mine = kTile * tg < cnt;   // this wave has tokens
+    issue_s(0);
+    issue_a(0, 0);
+    {   // the biases of this wave's rows; tokens from the list
+        const int bm = NM == 2 ? g : 0;
+        dma4(ldsI + 256u * wave, ex + A.off[MODE == 0 ? 2 + 3 * bm : 8] + (size_t)min(row0 + m, R - 1) * 4);
+        auto row = [&](int n) {
+            const int p = min(wave * kLoad + n, cnt - 1);
+            return (uint32_t)(MODE == 0 ? A.list_tok[base + p] : p) * (uint32_t)(S * kRec);
+        };
+#pragma unroll
+        for (int j = 0; j < kBLoads; ++j) {
+            const int i = min(64 * j + l, kLoad * kPieces - 1), n = i / kPieces;
+            boff[j] = row(n) + 16u * (i - n * kPieces);
         }
     }
+    issue_b(0, 0);
+    issue_a(1, 1);   // (S >= 2)
+    issue_b(1, 1);
+    const int p = kTile * tg + m;   // this lane's token
+    int slot = 0;
+    if constexpr (MODE == 1) slot = A.slot_of[base + min(p, cnt - 1)];
+    auto step = [&](auto bufc, int st) __attribute__((always_inline)) {
+        constexpr int buf = decltype(bufc)::value;
+        __builtin_amdgcn_sched_barrier(0);   // (products moved into the next step would hold two steps' operands)
+        // step st is in LDS (the next one's loads stay in flight)
+        if (st + 1 == S) dma_wait<0>();
+        else if (loads_b) dma_wait<kALoads + kBLoads>();
+        else dma_wait<kALoads>();
+        dma_barrier();
+        Operands ops;
+        if (mine) {
+            if (buf == 0) {
+                if (st % 4 == 0) {
+                    scales(st);
+                } else {
+#pragma unroll
+                    for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+                        for (int r = 0; r < kRG; ++r) sw4[mt][r][0] = sw4[mt][r][1];
+                }
+            }
+            read(buf, ops);
+        }
+        // every wave holds the step in registers: its buffers take step st + 2
+        dma_barrier();
+        if (buf == 0 && st % 4 == 0 && st + 4 < S) issue_s(st + 4);
+        if (st + 2 < S) {
+            issue_a(st + 2, buf);
+            issue_b(st + 2, buf);
+        }
+        if (mine) math(bufc, ops);
+    };
+    for (int st = 0; st < S; st += 2) {
+        step(std::integral_constant<int, 0>{}, st);
+        if (st + 1 < S) step(std::integral_constant<int, 1>{}, st + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if (bad) atomicOr(A.err, 1u);
+    if (!mine) return;
+    // Outputs: the lane holds rows 8 (i / 4) + 4 g + i % 4 of each row tile
+    // for its token.
+    auto bias = [&](int mt, int r, int q) {   // rows 8 q + 4 g .. of row tile r
+        const int rt = kRG * rg + r;
+        return *(const float4 *)(glds + 2 * (kLdsB + gemm_a(NM)) + gemm_s(NM) + 256 * rt + 128 * mt +
+                                 32 * q + 16 * g);
+    };
+    const int rt0 = rgrp * kRows + kRG * rg * kTile;   // the wave's first row
+    if constexpr (MODE == 0) {
+        // A row tile is a 32-block of h, half of it in each of a token's two
+        // lanes: lane g gets both halves of tile g and quantizes it. Rows past
+        // F are zeros.
+        const bool plain = A.act_plain != 0;   // g / (1 + e^-g) u: no limits, alpha 1, nothing added to u
+        const float limit = plain ? INFINITY : A.limit, alpha = plain ? 1.0f : A.alpha, one = plain ? 0.0f : 1.0f;
+        float hv[kRG][16];
+#pragma unroll
+        for (int r = 0; r < kRG; ++r)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 b0 = bias(0, r, q), b1 = bias(1, r, q);
+                const float gb[4] = {b0.x, b0.y, b0.z, b0.w}, ub[4] = {b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float gg = acc[0][r][4 * q + e] + gb[e];
+                    float uu = acc[NM - 1][r][4 * q + e] + ub[e];
+                    if (gg > limit) gg = limit;
+                    if (uu > limit) uu = limit;
+                    if (uu < -limit) uu = -limit;
+                    const float o = gg / (1.0f + expf(-alpha * gg)) * (uu + one);
+                    hv[r][4 * q + e] = rt0 + kTile * r < R ? o : 0.f;
+                }
+                __builtin_amdgcn_sched_barrier(0);   // (four at a time: registers)
+            }
+        static_assert(kRG == 2, "one row tile per lane of a token");
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        float v[32];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {   // tile 0's upper half of the lanes with tile 1's lower one
+            const v2u x = __builtin_amdgcn_permlane32_swap(__float_as_uint(hv[0][e]), __float_as_uint(hv[1][e]), false, false);
+            v[8 * (e >> 2) + (e & 3)] = __uint_as_float(x.x);
+            v[8 * (e >> 2) + 4 + (e & 3)] = __uint_as_float(x.y);
+        }
+        if (p < cnt) quant_block(v, A.hq + ((size_t)(base + p) * groups + rgrp) * kRec, kRG * rg + g);
+    } else {
+        if (p >= cnt) return;
+        float *out = A.ye + (size_t)slot * A.H + rt0 + 4 * g;
+#pragma unroll
+        for (int r = 0; r < kRG; ++r) {
+            if (rt0 + kTile * r >= R) break;   // wave-uniform: R is a multiple of the tile
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 b = bias(0, r, q);
+                *(float4 *)(out + kTile * r + 8 * q) = float4{acc[0][r][4 * q] + b.x, acc[0][r][4 * q + 1] + b.y,
+                                                              acc[0][r][4 * q + 2] + b.z, acc[0][r][4 * q + 3] + b.w};
+            }
+        }
+    }
 }
 
 }  // namespace
 
-// Assignments grouped by expert (offsets[E + 1], token and slot of each list
-// position) and their passes in the S_LIST scratch; E <= 4096.
+// Assignments grouped by expert (token and slot of each list position) and
+// their passes in the S_LIST scratch; E <= 4096.
 int launch_expert_lists(const int32_t *sel, int N, int E, int k, ExpertLists *out, hipStream_t s) {
     if (E > kPlistMaxE) return fail(MH_E_UNSUPPORTED, "expert lists: %d experts > %d", E, kPlistMaxE);
     void *pl;
-    MH_TRY(scratch(S_LIST, sizeof(int) * (2 * ((size_t)E + 1) + 3 * (size_t)N + (size_t)pass_max(N, E)), &pl));
-    int *offs = (int *)pl, *rank = offs + E + 1;
-    out->offs = offs;
+    const size_t np = (size_t)pass_max(N, E);
+    MH_TRY(scratch(S_LIST, sizeof(Pass) * np + sizeof(int) * (1 + 3 * (size_t)N), &pl));
+    Pass *passes = (Pass *)pl;
+    int *npass = (int *)(passes + np), *rank = npass + 1;
+    out->passes = passes;
+    out->npass = npass;
     out->list_tok = rank + N;
     out->slot_of = rank + 2 * (size_t)N;
-    out->poff = rank + 3 * (size_t)N;
-    out->pexp = out->poff + E + 1;
-    MH_LAUNCH("plist", k_plist_one, dim3(1), dim3(1024), 0, s, sel, N, E, k, rank, offs, out->list_tok, out->slot_of,
-              out->poff, out->pexp);
+    MH_LAUNCH("plist", k_plist_one, dim3(1), dim3(1024), 0, s, sel, N, E, k, rank, out->list_tok, out->slot_of, passes,
+              npass);
     return hip_check(hipGetLastError(), "expert lists launch");
 }
 
@@ -528,9 +605,8 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
     A.alpha = L.alpha;
     A.limit = L.limit;
     A.act_plain = L.act_plain;
-    A.offs = lists.offs;
-    A.poff = lists.poff;
-    A.pexp = lists.pexp;
+    A.passes = (const Pass *)lists.passes;
+    A.npass = lists.npass;
     A.list_tok = lists.list_tok;
     A.slot_of = lists.slot_of;
     A.bq = qx;
@@ -539,18 +615,15 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
     A.err = scale_err_dev;
 
     // a block for every pass that the assignments can make (those without one return)
-    auto grid = [&](int R) {
-        const int64_t nb = pass_max(N, E) * ((R + kRows - 1) / kRows);
-        return dim3((unsigned)((nb + 7) / 8 * 8));
-    };
+    auto grid = [&](int groups) { return dim3((unsigned)((pass_max(N, E) * groups + 7) / 8 * 8)); };
     if (xb) {
         const int64_t thr = (int64_t)n * 4 * k_steps(H);
         MH_LAUNCH("quant_x", k_quant_terms, dim3((unsigned)((thr + 255) / 256)), dim3(256), 0, s, xb, n, H, qx);
     }
     // gate/up over the quantized tokens, then down over the quantized h
-    MH_LAUNCH("moe_gu_mfma", k_moe_gemm<0>, grid(F), dim3(64 * kWaves), gemm_lds(2), s, A);
+    MH_LAUNCH("moe_gu_mfma", k_moe_gemm<0>, grid(k_steps(F)), dim3(64 * kWaves), gemm_lds(2), s, A);
     A.bq = qh;
-    MH_LAUNCH("moe_down_mfma", k_moe_gemm<1>, grid(H), dim3(64 * kWaves), gemm_lds(1), s, A);
+    MH_LAUNCH("moe_down_mfma", k_moe_gemm<1>, grid((H + kRows - 1) / kRows), dim3(64 * kWaves), gemm_lds(1), s, A);
     return hip_check(hipGetLastError(), "prefill MFMA launches");
 }
 

@@ -1,5 +1,5 @@
-"""The scaled-matrix-core prefill at the edges of its tiles (16 rows and tokens,
-passes of up to 8 token tiles, K steps of 128 columns, blocks of 128 rows)
+"""The scaled-matrix-core prefill at the edges of its tiles (32 rows and tokens,
+passes of up to 2 token tiles, K steps of 128 columns, blocks of 128 rows)
 against the per-assignment GEMVs on the same weights."""
 import numpy as np
 import pytest
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # uniform error 2^-12 / sqrt(3) of it, and that value is ~2.2 rms of a normal
 # block: 3.1e-4 of a product sum, once in gate/up and once in down.
 TOL = 6.2e-4
-COUNTS = [1, 0, 15, 16, 17, 127, 128, 129, 257]   # tokens of each expert
+COUNTS = [1, 0, 16, 31, 32, 33, 63, 64, 65, 129, 257]   # tokens of each expert
 
 
 @pytest.mark.parametrize("hidden,ffn,plain", [(64, 64, False), (64, 192, True), (192, 320, False), (256, 128, False),
@@ -27,7 +27,7 @@ def test_gemm_edges(mh, path_switch, hidden, ffn, plain):
     w, s, b, nw = synth.host_router(shape, keys, 0)
     lay = MoELayer.host(shape, ex, w, s, b, nw)
     rng = np.random.default_rng(hidden + ffn)
-    flat = np.concatenate([np.repeat(np.arange(len(COUNTS)), COUNTS), [-1, len(COUNTS)]]).astype(np.int32)
+    flat = np.concatenate([np.repeat(np.arange(len(COUNTS)), COUNTS), [-1, len(COUNTS), -1]]).astype(np.int32)
     sel = rng.permutation(flat).reshape(-1, 2)   # a token may hold one expert twice: two assignments
     n = len(sel)
     wt = rng.uniform(0.5, 1.0, (n, 2)).astype(np.float32)
