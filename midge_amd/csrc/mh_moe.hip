@@ -569,21 +569,20 @@ __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
 }
 
 // The router of a prefill of more than kCRTok tokens in one launch: RMSNorm,
-// router logits, top-k and weights of TB tokens per block, and the normed
-// input either as f32 rows (xb) or as the matrix product's records (rec,
-// mh_fp6.cuh), so that it is not written and read again in between.
-//   A lane keeps its 16-element chunks of the tokens' xb in registers and the
-//   waves walk the experts' rows (L2 hits), one row ahead. LDS holds xb with
-//   4 floats after every 32 (a lane's chunks and blocks fall in distinct
-//   banks).
-//   Two tokens share a row's conversions from 1024 tokens on; below that one
-//   token per block keeps more blocks in flight.
+// router logits, top-k and weights, and the normed input either as f32 rows
+// (xb) or as the matrix product's records (rec, mh_fp6.cuh), so that it is not
+// written and read again in between. W waves per token, each with the whole
+// token in registers (a lane holds three chunks of 16 elements) and every
+// W-th group of four experts, whose rows it reads one ahead (a block's waves
+// share them in the L1) and whose sums it reduces together. The two lanes
+// that hold a 32-block of x exchange halves to quantize it.
+//   W is 8, 4, 2 or 1 as the tokens come to fill the chip's 1024 SIMDs twice.
 // (norm, one GEMV per token, top-k and the quantizer as four launches took 15
 // + 121 + 6 + 9 us for 2000 tokens of a 32-expert layer and 5 + 33 + 5 + 5 for
 // 512, mostly for reading the router's rows and the norm's output once per
-// token and block; this takes 47 and 14 us.)
-constexpr int kRTThreads = 512;
-constexpr int kRTPad = kCRMaxH / 32 * 36;   // floats of a padded row
+// token and block; this takes 33 and 15 us, and 47 and 14 with two tokens or
+// one per block and the norm shared through LDS.)
+constexpr int kRTWaves = 8;   // waves per block
 
 struct RouteTokArgs {
     const float *x;        // [n][H]
@@ -597,20 +596,19 @@ struct RouteTokArgs {
     uint8_t *rec;          // records out, or null
     int32_t *sel;          // [n][k] out
     float *w;              // [n][k] out
+    int W;                 // waves per token (1, 2, 4 or 8)
 };
 
-template <int PER, int TB>
-__global__ void __launch_bounds__(kRTThreads, TB == 1 ? 4 : 2) k_route_tokens(RouteTokArgs A) {
+template <int PER>
+__global__ void __launch_bounds__(64 * kRTWaves, 4) k_route_tokens(RouteTokArgs A) {
 #pragma clang fp contract(off)
-    constexpr int kW = kRTThreads / 64, kV = kCRMaxH / kRTThreads;
-    constexpr int CE = mh_chunk<MH_DT_Q8R>::E, kC = cr_chunks<MH_DT_Q8R>();
-    static_assert(CE == 16, "a 32-block holds two chunks");
-    __shared__ float part[kW][TB];
-    __shared__ __attribute__((aligned(16))) float s_xb[TB][kRTPad];
-    __shared__ float s_rl[TB][64 * PER];
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    constexpr int CE = mh_chunk<MH_DT_Q8R>::E, kC = cr_chunks<MH_DT_Q8R>(), kRows = 4;
+    static_assert(CE == 16 && kC == 3, "a 32-block is two lanes' chunks");
+    __shared__ float s_rl[kRTWaves][64 * PER];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int H = A.H, E = A.E, C = H / CE;
-    const int t0 = (int)blockIdx.x * TB, nt = min(TB, A.n - t0);
+    const int sub = wave % A.W, own = wave / A.W, tok = (int)blockIdx.x * (kRTWaves / A.W) + own;
+    const int t = min(tok, A.n - 1);   // (past the last token: the last again, nothing written)
     const mh_rsrc rr = gemv_rsrc(A.rw, (uint32_t)E * (uint32_t)H);
     mh_u4 q[kC];
     auto load_row = [&](int e) __attribute__((always_inline)) {
@@ -619,90 +617,98 @@ __global__ void __launch_bounds__(kRTThreads, TB == 1 ? 4 : 2) k_route_tokens(Ro
         for (int j = 0; j < kC; ++j)   // past the row: its last chunk again (xb is zero there)
             q[j] = __builtin_amdgcn_raw_buffer_load_b128(rr, row + 16u * (uint32_t)min(lane + 64 * j, C - 1), 0, 0);
     };
-    float v[TB][kV];
+    const float *xt = A.x + (size_t)t * H;
+    const bool vec = ((uintptr_t)xt | (uintptr_t)A.nw) % 16 == 0;   // wave-uniform
+    auto load16 = [&](const float *p, float (&v)[CE]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < TB; ++b) {
-        const float *xt = A.x + (size_t)min(t0 + b, A.n - 1) * H;
+        for (int i = 0; i < CE; i += 4) {
+            float4 a;
+            if (vec) a = *(const float4 *)(p + i);
+            else a = float4{p[i], p[i + 1], p[i + 2], p[i + 3]};
+            v[i] = a.x; v[i + 1] = a.y; v[i + 2] = a.z; v[i + 3] = a.w;
+        }
+    };
+    float xr[kC][CE], nr[kC][CE];
+#pragma unroll
+    for (int j = 0; j < kC; ++j) load16(xt + min(lane + 64 * j, C - 1) * CE, xr[j]);
+#pragma unroll
+    for (int j = 0; j < kC; ++j) load16(A.nw + min(lane + 64 * j, C - 1) * CE, nr[j]);
+    load_row(kRows * sub);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < kC; ++j) {
+        const bool in = lane + 64 * j < C;
         float s = 0.f;
 #pragma unroll
-        for (int u = 0; u < kV; ++u) {
-            const int r = tid + kRTThreads * u;
-            v[b][u] = r < H ? xt[r] : 0.f;
-            s = __builtin_fmaf(v[b][u], v[b][u], s);
+        for (int i = 0; i < CE; ++i) {
+            xr[j][i] = in ? xr[j][i] : 0.f;
+            s = __builtin_fmaf(xr[j][i], xr[j][i], s);
         }
-        s = mh_wave_sum(s);
-        if (lane == 0) part[wave][b] = s;
+        ss += s;
     }
-    load_row(wave);
-    __syncthreads();
+    ss = mh_wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)H + A.eps);
 #pragma unroll
-    for (int b = 0; b < TB; ++b) {
-        float ss = 0.f;
+    for (int j = 0; j < kC; ++j) {
+        const int c = lane + 64 * j;
 #pragma unroll
-        for (int i = 0; i < kW; ++i) ss += part[i][b];
-        const float inv = 1.0f / sqrtf(ss / (float)H + A.eps);
+        for (int i = 0; i < CE; ++i) xr[j][i] = xr[j][i] * inv * nr[j][i];
+        if (c >= C) {   // (a norm weight may be infinite)
 #pragma unroll
-        for (int u = 0; u < kV; ++u) {
-            const int r = tid + kRTThreads * u;
-            if (r < H) {
-                const float xbv = v[b][u] * inv * A.nw[r];
-                s_xb[b][r + (r >> 5) * 4] = xbv;
-                if (A.xb && b < nt) A.xb[(size_t)(t0 + b) * H + r] = xbv;
-            }
+            for (int i = 0; i < CE; ++i) xr[j][i] = 0.f;
+        } else if (A.xb && sub == 0 && tok < A.n) {
+            float *o = A.xb + (size_t)t * H + c * CE;
+#pragma unroll
+            for (int i = 0; i < CE; i += 4) *(float4 *)(o + i) = float4{xr[j][i], xr[j][i + 1], xr[j][i + 2], xr[j][i + 3]};
         }
     }
-    __syncthreads();
-    float xr[TB][kC][CE];
+    for (int e0 = kRows * sub; e0 < E; e0 += kRows * A.W) {
+        float acc[kRows];
 #pragma unroll
-    for (int b = 0; b < TB; ++b)
+        for (int r = 0; r < kRows; ++r) {
+            mh_u4 cur[kC];
 #pragma unroll
-        for (int j = 0; j < kC; ++j) {
-            const int c = lane + 64 * j;
-            const float *src = s_xb[b] + min(c, C - 1) * CE + (min(c, C - 1) >> 1) * 4;
+            for (int j = 0; j < kC; ++j) cur[j] = q[j];
+            load_row(r + 1 < kRows ? e0 + r + 1 : e0 + kRows * A.W);
+            acc[r] = 0.f;
 #pragma unroll
-            for (int i = 0; i < CE; i += 4) {
-                const float4 a = *(const float4 *)(src + i);
-                xr[b][j][i] = c < C ? a.x : 0.f;
-                xr[b][j][i + 1] = c < C ? a.y : 0.f;
-                xr[b][j][i + 2] = c < C ? a.z : 0.f;
-                xr[b][j][i + 3] = c < C ? a.w : 0.f;
-            }
+            for (int j = 0; j < kC; ++j) acc[r] += mh_dot_chunk<MH_DT_Q8R>(cur[j], xr[j]);
         }
-    for (int e = wave; e < E; e += kW) {
-        mh_u4 cur[kC];
 #pragma unroll
-        for (int j = 0; j < kC; ++j) cur[j] = q[j];
-        load_row(e + kW);
+        for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-        for (int b = 0; b < TB; ++b) {
-            float acc = 0.f;
-#pragma unroll
-            for (int j = 0; j < kC; ++j) acc += mh_dot_chunk<MH_DT_Q8R>(cur[j], xr[b][j]);
-            acc = mh_wave_sum(acc);
-            if (lane == 0) s_rl[b][e] = acc * A.rs[e];
-        }
+            for (int r = 0; r < kRows; ++r) acc[r] += __shfl_xor(acc[r], o, 64);
+        const float mine = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
+        if (lane < kRows && e0 + lane < E) s_rl[own][e0 + lane] = mine * A.rs[e0 + lane];
     }
     __syncthreads();
-    if (wave < nt) {
-        const size_t o = (size_t)(t0 + wave) * A.k;
-        wave_topk_token<PER>(s_rl[wave], A.rb, E, A.k, A.router_norm, A.unfilled, A.sel + o, A.w + o, nullptr);
-    } else if (A.rec && wave >= TB) {   // the other waves quantize
+    if (tok >= A.n) return;   // wave-uniform
+    if (A.rec && sub == A.W - 1) {
         const int nst = k_steps(H), nb = 4 * nst;
-        for (int u = tid - 64 * TB; u < nt * nb; u += kRTThreads - 64 * TB) {
-            const int b = u / nb, blk = u - b * nb;
-            float vb[32];
+        uint8_t *rec = A.rec + (size_t)t * nst * kRec;
+        const bool odd = lane & 1;
+        // block lane / 2 of 32 (chunks 0) by the even lane, block 32 + lane / 2
+        // (chunks 1) by the odd one, then 64 + lane / 2 by the even one
+        float v[32];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 a = *(const float4 *)(s_xb[b] + min(blk, H / 32 - 1) * 36 + 4 * j);
-                const bool in = 32 * blk < H;
-                vb[4 * j + 0] = in ? a.x : 0.f;
-                vb[4 * j + 1] = in ? a.y : 0.f;
-                vb[4 * j + 2] = in ? a.z : 0.f;
-                vb[4 * j + 3] = in ? a.w : 0.f;
-            }
-            quant_block(vb, A.rec + ((size_t)(t0 + b) * nst + (blk >> 2)) * kRec, blk & 3);
+        for (int i = 0; i < CE; ++i) {
+            const float other = dpp_x1(odd ? xr[0][i] : xr[1][i]);
+            v[i] = odd ? other : xr[0][i];
+            v[16 + i] = odd ? xr[1][i] : other;
         }
+        int b = (lane >> 1) + (odd ? 32 : 0);
+        if (b < nb) quant_block(v, rec + (b >> 2) * kRec, b & 3);
+#pragma unroll
+        for (int i = 0; i < CE; ++i) {
+            v[16 + i] = dpp_x1(xr[2][i]);
+            v[i] = xr[2][i];
+        }
+        b = 64 + (lane >> 1);
+        if (!odd && b < nb) quant_block(v, rec + (b >> 2) * kRec, b & 3);
     }
+    if (sub != 0) return;
+    const size_t o = (size_t)t * A.k;
+    wave_topk_token<PER>(s_rl[own], A.rb, E, A.k, A.router_norm, A.unfilled, A.sel + o, A.w + o, nullptr);
 }
 
 // zeroes n words (a fill kernel: no memset node in a caller's graph)
@@ -948,13 +954,14 @@ int launch_route_tokens(const DevLayer &L, const float *x, int n, float *xb, uin
     A.rec = rec;
     A.sel = sel;
     A.w = w;
-    auto go = [&](auto one, auto two) {
-        if (n < 1024) MH_LAUNCH("route_tokens", one, dim3((unsigned)n), dim3(kRTThreads), 0, s, A);
-        else MH_LAUNCH("route_tokens", two, dim3((unsigned)((n + 1) / 2)), dim3(kRTThreads), 0, s, A);
+    A.W = n >= 2048 ? 1 : n >= 1024 ? 2 : n >= 512 ? 4 : 8;
+    const int per = kRTWaves / A.W;   // tokens per block
+    auto go = [&](auto kern) {
+        MH_LAUNCH("route_tokens", kern, dim3((unsigned)((n + per - 1) / per)), dim3(64 * kRTWaves), 0, s, A);
     };
-    if (L.n_experts <= 128) go(k_route_tokens<2, 1>, k_route_tokens<2, 2>);
-    else if (L.n_experts <= 256) go(k_route_tokens<4, 1>, k_route_tokens<4, 2>);
-    else go(k_route_tokens<kMaxExperts / 64, 1>, k_route_tokens<kMaxExperts / 64, 2>);
+    if (L.n_experts <= 128) go(k_route_tokens<2>);
+    else if (L.n_experts <= 256) go(k_route_tokens<4>);
+    else go(k_route_tokens<kMaxExperts / 64>);
     return hip_check(hipGetLastError(), "route launch");
 }
 
