@@ -119,12 +119,31 @@ k_xdigits(const float *__restrict__ X, int K, int batch, uint8_t *__restrict__ x
     const int n = cl >> 4, cn = cl & 15, KC = K >> 6;
     const bool live = c < batch;
     const float *x = X + (size_t)(live ? c : 0) * K;
-    float m = 0.f;
-    if (live)
-        for (int k = threadIdx.x; k < K; k += blockDim.x) m = fmaxf(m, fabsf(x[k]));
+    // a thread's first 16 elements stay in registers (all of K up to 4096)
+    const int np = KC * 4;
+    const bool vec = (uintptr_t)x % 16 == 0;
+    auto load16 = [&](int p, float (&v)[16]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 16; j += 4) {
+            float4 a;
+            if (vec) a = *(const float4 *)(x + p * 16 + j);
+            else a = float4{x[p * 16 + j], x[p * 16 + j + 1], x[p * 16 + j + 2], x[p * 16 + j + 3]};
+            v[j] = a.x; v[j + 1] = a.y; v[j + 2] = a.z; v[j + 3] = a.w;
+        }
+    };
+    float v0[16] = {}, m = 0.f;
     bool bad = false;
     if (live)
-        for (int k = threadIdx.x; k < K; k += blockDim.x) bad |= !__builtin_isfinite(x[k]);
+        for (int p = threadIdx.x; p < np; p += blockDim.x) {
+            float v[16];
+            load16(p, v);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                m = fmaxf(m, fabsf(v[j]));
+                bad |= !__builtin_isfinite(v[j]);
+                if (p == (int)threadIdx.x) v0[j] = v[j];
+            }
+        }
     m = __builtin_isfinite(m) ? m : __builtin_inff();
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     const bool anybad = __syncthreads_or(bad);
@@ -134,8 +153,9 @@ k_xdigits(const float *__restrict__ X, int K, int batch, uint8_t *__restrict__ x
     int e = 0;
     if (m > 0.f && !anybad) (void)frexpf(m, &e);   // 2^(e-1) <= m < 2^e
     if (threadIdx.x == 0) shift[c] = anybad ? kQ8NonFinite : e - 22;
-    for (int p = threadIdx.x; p < KC * 4; p += blockDim.x) {
+    for (int p = threadIdx.x; p < np; p += blockDim.x) {
         const int kc = p >> 2, kg = p & 3;
+        if (p != (int)threadIdx.x && live && !anybad) load16(p, v0);
         uint32_t dw[3][4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -143,7 +163,7 @@ k_xdigits(const float *__restrict__ X, int K, int batch, uint8_t *__restrict__ x
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 int q = 0;
-                if (live && !anybad) q = (int)rintf(ldexpf(x[p * 16 + 4 * j + i], 22 - e));   // |q| <= 2^22
+                if (live && !anybad) q = (int)rintf(ldexpf(v0[4 * j + i], 22 - e));   // |q| <= 2^22
                 const int d2 = ((q + 128) & 255) - 128;
                 const int q1 = (q - d2) >> 8;
                 const int d1 = ((q1 + 128) & 255) - 128;
@@ -332,8 +352,10 @@ k_gemm_q8r(const int8_t *__restrict__ W, const float *__restrict__ S, const uint
 // instead of once per wave). The steps run on across passes: the next pass's
 // first loads fly under this one's last steps. Up to 64 columns meet each
 // weight byte. (lm_head 201088 x 2880 at batch 32: 187 us with each wave
-// reading its digits from L2 and its rows through registers, 144 us this way,
-// 4.2 TB/s in the kernel; the digits had been three times the weights' bytes.)
+// reading its digits from L2 and its rows through registers, 144 us with both
+// in LDS, 137 us with a step's LDS reads ahead of its loads and the digits
+// formed in registers (10 -> 5 us); 4.3 TB/s in the kernel. The digits had
+// been three times the weights' bytes.)
 // LDS: rows [3][wave][tile][16][8] 16-byte chunks, chunk c of row r at slot
 // c ^ (r % 8) (a read's 8 rows then fall in distinct banks); digits
 // [2][chunk][digit][column tile][64] words as they lie in memory.
@@ -415,25 +437,41 @@ k_gemm_q8r_rows(const int8_t *__restrict__ W, const float *__restrict__ S, const
 #pragma unroll
                 for (int d = 0; d < 3; ++d) acc[m][t][d] = mh_i4{0, 0, 0, 0};
     };
-    auto math = [&](auto mtc, int chunks, const uint8_t *la, const uint8_t *lb) __attribute__((always_inline)) {
+    // a step's chunks read ahead of its loads: both, where the registers hold them
+    constexpr int kAhead = NT <= 3 ? 2 : 1;
+    struct Operands {
+        mh_u4 a[2][kQ8MT], b[2][3][NT];
+    };
+    auto read = [&](auto mtc, int h0, int h1, const uint8_t *la, const uint8_t *lb, Operands &o)
+                    __attribute__((always_inline)) {
+        constexpr int M = decltype(mtc)::value;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (h < h0 || h >= h1) continue;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                o.a[h][m] = *(const mh_u4 *)(la + m * kQ8TileLds + 128 * i + 16 * ((4 * h + g) ^ (i & 7)));
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    o.b[h][d][t] = *(const mh_u4 *)(lb + ((h * 3 + d) * NT + t) * 1024 + 16 * lane);
+        }
+    };
+    auto math = [&](auto mtc, int chunks, const uint8_t *la, const uint8_t *lb, Operands &o) __attribute__((always_inline)) {
         constexpr int M = decltype(mtc)::value;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (h >= chunks) break;   // uniform
-            mh_u4 a[M];
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-                a[m] = *(const mh_u4 *)(la + m * kQ8TileLds + 128 * i + 16 * ((4 * h + g) ^ (i & 7)));
+            if (h >= kAhead) read(mtc, h, h + 1, la, lb, o);
 #pragma unroll
             for (int d = 0; d < 3; ++d)
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const mh_u4 b = *(const mh_u4 *)(lb + ((h * 3 + d) * NT + t) * 1024 + 16 * lane);
+                for (int t = 0; t < NT; ++t)
 #pragma unroll
                     for (int m = 0; m < M; ++m)
-                        acc[m][t][d] =
-                            __builtin_amdgcn_mfma_i32_16x16x64_i8((mh_i4)a[m], (mh_i4)b, acc[m][t][d], 0, 0, 0);
-                }
+                        acc[m][t][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8((mh_i4)o.a[h][m], (mh_i4)o.b[h][d][t],
+                                                                             acc[m][t][d], 0, 0, 0);
         }
     };
     auto store = [&](int m, int tile) __attribute__((always_inline)) {
@@ -495,14 +533,20 @@ k_gemm_q8r_rows(const int8_t *__restrict__ W, const float *__restrict__ S, const
         else if (left == 2) dma_wait<2>();
         else dma_wait<0>();
         dma_barrier();
+        // the operands' reads go first: they run while the loads, which wait
+        // for the load path, are issued (a last lone chunk reads a second one
+        // that is not multiplied)
+        const uint8_t *la = qlds + ab * kQ8RowsLds + wave * (kQ8MT * kQ8TileLds);
+        const uint8_t *lb = qlds + 3 * kQ8RowsLds + (it & 1) * q8_digits_lds(NT);
+        Operands ops;
+        if (mine == 2) read(std::integral_constant<int, 2>{}, 0, kAhead, la, lb, ops);
+        else if (mine == 1) read(std::integral_constant<int, 1>{}, 0, kAhead, la, lb, ops);
         const int nst = st + 1 == ST ? 0 : st + 1;
         if (it + 1 < total) issue_b(nst, (it + 1) & 1);
         left = it + 2 < total ? issue_a(ab == 0 ? 2 : ab - 1) : 0;
-        const uint8_t *la = qlds + ab * kQ8RowsLds + wave * (kQ8MT * kQ8TileLds);
-        const uint8_t *lb = qlds + 3 * kQ8RowsLds + (it & 1) * q8_digits_lds(NT);
         const int chunks = min(2, KC - 2 * st);
-        if (mine == 2) math(std::integral_constant<int, 2>{}, chunks, la, lb);
-        else if (mine == 1) math(std::integral_constant<int, 1>{}, chunks, la, lb);
+        if (mine == 2) math(std::integral_constant<int, 2>{}, chunks, la, lb, ops);
+        else if (mine == 1) math(std::integral_constant<int, 1>{}, chunks, la, lb, ops);
         if (nst == 0) {
             const int t0 = pass_beg(pass) + wave;
             if (mine > 0) store(0, t0);
