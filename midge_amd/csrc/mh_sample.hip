@@ -42,9 +42,12 @@
 //                   reaches topp * den by a margin that covers the f32
 //                   rounding; p >= RN(lower edge / den) holds every token of
 //                   those bins, division being monotone) and gathers its
-//                   tokens with p >= T. Last block: if they fit (<= kCap)
-//                   they are sorted in LDS (bitonic, by falling p then id),
-//                   scanned in f64, and the nucleus and the pick read off.
+//                   tokens with p >= T. Last block: if they fit (<= kCap), a
+//                   histogram of their p finds the bins where the running sum
+//                   crosses topp and u * cum, and only those bins' tokens are
+//                   ranked; or, if a bin is too full, all are sorted in LDS
+//                   (bitonic, by falling p then id), scanned in f64, and the
+//                   nucleus and the pick read off.
 //                   Otherwise (a flat distribution, or topp close to 1,
 //                   where every block has stored p instead) an exact radix
 //                   select over all V: four histogram levels over p's bits
@@ -627,6 +630,157 @@ __device__ bool pick_sorted(const Probs &P, int cnt, int V, float topp, float u,
     __syncthreads();
     if (t == 0) *out = L.sort.id[s_pick];
     return true;
+}
+
+// pick_sorted for more candidates than are ranked one by one, without
+// ordering them all: a histogram of their p over kLB bins (64 to an octave)
+// finds the bin where the running sum from the top crosses topp; the
+// candidates of that bin alone are ranked, which gives the nucleus's end and
+// its sum, and the same again finds the draw. The masses are integers of
+// 2^-63 (p <= 1; exact for p >= 2^-40, whose last bit is 2^-63 or more), so
+// the sums do not depend on the order of the additions. 0: no pick (nothing
+// written): a bin holds more candidates than are ranked, or p lies below the
+// bins; the sort decides. (With the bitonic sort of all candidates the select
+// launch took 38.6 us for a few thousand of 201088 tokens, with this 24.9.)
+constexpr int kLB = 4096, kLBRank = 512;
+struct ListLds {   // over SelLds::sort.pre
+    unsigned long long mass[kLB];
+    unsigned cnt[kLB];
+    uint64_t key[kLBRank];
+};
+static_assert(sizeof(ListLds) <= sizeof(double) * kCap && kLB % kSelThreads == 0, "the histogram's LDS");
+__device__ int pick_listed(const Probs &P, int cnt, int V, float topp, float u, SelLds &L, int32_t *out) {
+    __shared__ int s_bin, s_m, s_n;
+    __shared__ unsigned long long s_above, s_key;
+    __shared__ double s_x;
+    __shared__ uint32_t s_lo;
+    ListLds &H = *(ListLds *)L.sort.pre;
+    constexpr int kPer = kCap / kSelThreads, kBins = kLB / kSelThreads;
+    constexpr double kUnit = 9223372036854775808.0;   // 2^63
+    const int t = threadIdx.x;
+    uint32_t bits[kPer];
+    int id[kPer];
+    if (t == 0) s_lo = 0xFFFFFFFFu;
+    for (int b = t; b < kLB; b += kSelThreads) {
+        H.mass[b] = 0ull;
+        H.cnt[b] = 0u;
+    }
+    __syncthreads();
+    uint32_t lo = 0xFFFFFFFFu;
+    bool bad = false;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int i = t + q * kSelThreads;
+        id[q] = i < cnt ? L.sort.id[i] : -1;
+        const float p = i < cnt ? P(id[q]) : 0.f;
+        bits[q] = __float_as_uint(p);
+        if (i < cnt) {
+            bad |= !(p >= 0.f && p <= 1.f);
+            lo = min(lo, bits[q]);
+        }
+    }
+    atomicMin(&s_lo, lo);
+    if (__syncthreads_or(bad)) return 0;
+    const uint32_t b0 = s_lo >> 17;
+    if ((0x3F800000u >> 17) - b0 >= (uint32_t)kLB) return 0;   // block-uniform
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+        if (id[q] >= 0) {
+            const uint32_t b = (bits[q] >> 17) - b0;
+            atomicAdd(&H.mass[b], (unsigned long long)((double)__uint_as_float(bits[q]) * kUnit));
+            atomicAdd(&H.cnt[b], 1u);
+        }
+    __syncthreads();
+    // thread t holds bins kLB - 1 - kBins t and down: the mass above each
+    // group, and the whole (a scan of integers through two 32-bit halves
+    // would wrap: 64-bit sums by shuffles)
+    unsigned long long own[kBins], run = 0ull;
+#pragma unroll
+    for (int j = 0; j < kBins; ++j) {
+        own[j] = H.mass[kLB - 1 - (kBins * t + j)];
+        run += own[j];
+    }
+    __shared__ unsigned long long ws[kSelThreads / 64];
+    unsigned long long inc = run;
+    const int lane = t & 63, w = t >> 6;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long n = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += n;
+    }
+    if (lane == 63) ws[w] = inc;
+    __syncthreads();
+    unsigned long long above = inc - run;
+    for (int i = 0; i < w; ++i) above += ws[i];
+    // The candidate where the running sum first reaches x (f64 compares, as the
+    // sort's): its bin, then its place there. Its id, its key and the sum up
+    // to and with it; -1 if no bin reaches x, -2 if the bin is too full.
+    auto find = [&](double x, int *pid, uint64_t *pkey, double *sum) -> int {
+        if (t == 0) {
+            s_bin = -1;
+            s_m = 0;
+            s_n = INT32_MAX;
+        }
+        __syncthreads();
+        unsigned long long a = above;
+#pragma unroll
+        for (int j = 0; j < kBins; ++j) {
+            if (own[j] && (double)a / kUnit < x && (double)(a + own[j]) / kUnit >= x) {
+                s_bin = kLB - 1 - (kBins * t + j);   // one thread: the sums tile
+                s_above = a;
+            }
+            a += own[j];
+        }
+        __syncthreads();
+        const int bin = s_bin;
+        if (bin < 0) return -1;
+        const int m = (int)H.cnt[bin];
+        if (m > kLBRank) return -2;
+        // the bin's candidates by falling p then id
+#pragma unroll
+        for (int q = 0; q < kPer; ++q)
+            if (id[q] >= 0 && (int)((bits[q] >> 17) - b0) == bin)
+                H.key[atomicAdd(&s_m, 1)] = ((uint64_t)bits[q] << 32) | (uint64_t)(~(uint32_t)id[q]);
+        __syncthreads();
+        const uint64_t k = t < m ? H.key[t] : 0ull;
+        int rank = 0;
+        double to = 0;   // the sum up to and with this candidate
+        if (t < m) {
+            unsigned long long sum_to = s_above;
+            for (int j = 0; j < m; ++j) {
+                const uint64_t kj = H.key[j];
+                if (kj < k) continue;
+                sum_to += (unsigned long long)((double)__uint_as_float((uint32_t)(kj >> 32)) * kUnit);
+                rank += kj > k ? 1 : 0;
+            }
+            to = (double)sum_to / kUnit;
+            if (to >= x) atomicMin(&s_n, rank);
+        }
+        __syncthreads();
+        const int place = s_n;
+        if (t < m && rank == place) {
+            s_key = k;
+            s_x = to;
+        }
+        __syncthreads();
+        *pkey = s_key;
+        *pid = (int)~(uint32_t)s_key;
+        *sum = s_x;
+        __syncthreads();
+        return place;
+    };
+    int last, pick;
+    uint64_t klast, kpick;
+    double cum, dummy;
+    const int n = find((double)topp, &last, &klast, &cum);
+    if (n < 0) return 0;
+    const float r = u * (float)cum;
+    // r <= 0: the first token of the order; a draw past the nucleus: its last
+    const int k = find(r <= 0.f ? 1e-300 : (double)r, &pick, &kpick, &dummy);
+    if (k == -2) return 0;
+    if (k < 0 || kpick < klast) pick = last;
+    if (t == 0) *out = pick;
+    return 1;
 }
 
 // The nucleus and the pick over the whole vocabulary (radix select).
@@ -1265,6 +1419,8 @@ __global__ void __launch_bounds__(kSelThreads) k_samp_select(const float *__rest
     const int cnt = (int)ld_agent(&ws->nsel);
     if (cnt >= 1 && cnt <= kCap) {
         for (int j = t; j < cnt; j += kSelThreads) L.sort.id[j] = ld_agent(&ws->cand[j]);
+        __syncthreads();
+        if (cnt > kRankMax && pick_listed(P, cnt, V, topp, u, L, out)) return;
         __syncthreads();
         if (pick_sorted(P, cnt, V, topp, u, L, out, false)) return;
         __syncthreads();
