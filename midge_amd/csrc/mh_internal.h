@@ -79,7 +79,8 @@ int async_flag(AsyncFlag id, const char *msg, unsigned **dev);
 //   BATCH_GEMV  decode steps of several tokens on the per-assignment GEMVs
 //               instead of the expert-grouped matrix-core kernels
 //   SPLIT_ROUTE a stack decode's layer boundary (combine, norm, router,
-//               top-k) as three launches instead of k_combine_route
+//               top-k), or a prefill's router, as three launches instead of
+//               k_combine_route or k_route_tokens
 enum Switch { SW_NO_MFMA = 0, SW_NO_FUSED, SW_ATTN_SPLIT, SW_COOP, SW_Q8_NO_ROWS, SW_BATCH_GEMV, SW_SPLIT_ROUTE, SW_COUNT };
 bool sw(Switch s);
 
