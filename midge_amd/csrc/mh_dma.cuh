@@ -10,6 +10,11 @@
 // make the wait longer), and dma_barrier then makes every wave's visible. A
 // buffer is loaded again only after a barrier that follows its last reads,
 // and the last loads are waited for before the block ends.
+//
+// The LDS address is in m0, which the loads take as an operand: the compiler
+// sets it, and knows of every value that it holds (a statement that wrote m0
+// itself would change it behind the compiler's back, and naming a reserved
+// register as clobbered does not keep a value across it).
 #pragma once
 
 #include "mh_internal.h"
@@ -21,11 +26,11 @@ __device__ __forceinline__ uint32_t lds_offset(const void *p) {
 }
 __device__ __forceinline__ void dma16(uint32_t lds, const uint8_t *p) {
     lds = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t lds, const uint8_t *p) {
     lds = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 __device__ __forceinline__ uint64_t uniform_addr(const uint8_t *p) {
     const uint64_t a = (uint64_t)p;
@@ -36,12 +41,12 @@ __device__ __forceinline__ uint64_t uniform_addr(const uint8_t *p) {
 // wait states before the load: its scalar operands may come from a vector
 // instruction, and the compiler cannot see that it reads them.)
 __device__ __forceinline__ void dma16(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(__builtin_amdgcn_readfirstlane(lds)),
                  "v"(off), "s"(uniform_addr(base))
                  : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+    asm volatile("s_nop 4\n\tglobal_load_lds_dword %1, %2" ::"{m0}"(__builtin_amdgcn_readfirstlane(lds)),
                  "v"(off), "s"(uniform_addr(base))
                  : "memory");
 }
