@@ -444,7 +444,7 @@ struct CombineRouteArgs {
     int32_t *sel;          // [n][k] out
     float *w;              // [n][k] out
     uint32_t *usage;       // [E] or null
-    GroupTab tab;          // out
+    GroupTab tab;          // out (null order: none)
     unsigned *cnt;         // [n + 1] arrival counters
 };
 
@@ -549,6 +549,7 @@ __global__ void __launch_bounds__(1024) k_combine_route(CombineRouteArgs A) {
     if (wave == 0)
         wave_topk_token<PER>(A.rl + (size_t)t * E, A.rb, E, k, A.router_norm, A.unfilled, A.sel + (size_t)t * k,
                              A.w + (size_t)t * k, A.usage);
+    if (A.tab.order == nullptr) return;   // grid-uniform
     // the launch's last ranked token writes the table of groups
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -880,17 +881,30 @@ bool combine_route_ok(const DevLayer &L, int n) {
            (uint64_t)L.n_experts * (uint64_t)L.hidden * (L.router.dt == MH_DT_Q8R ? 1u : 4u) < (1ull << 32);
 }
 
-int launch_combine_route(const DevLayer &L, float *x, const float *ye, const float *wprev, int n, float *xb,
-                         float *rl, int32_t *sel, float *w, uint32_t *usage, const GroupTab &tab, int unfilled,
-                         hipStream_t s) {
-    if (!combine_route_ok(L, n)) return MH_E_UNSUPPORTED;
-    void *cp = nullptr;
+// Its arrival counters; null where the memory cap leaves none (the caller
+// routes in separate launches, which need none).
+int route_counters(unsigned **cnt, hipStream_t s) {
+    void *p = nullptr;
     bool fresh = false;
-    MH_TRY(scratch(S_CROUTE, sizeof(unsigned) * (kCRTok + 1), &cp, &fresh));
+    *cnt = nullptr;
+    const int rc = scratch(S_CROUTE, sizeof(unsigned) * (kCRTok + 1), &p, &fresh);
+    if (rc == MH_E_NOMEM) {
+        clear_error();
+        return MH_OK;
+    }
+    MH_TRY(rc);
     if (fresh) {
-        MH_LAUNCH("zero_counters", k_zero_u32, dim3(1), dim3(128), 0, s, (uint32_t *)cp, kCRTok + 1);
+        MH_LAUNCH("zero_counters", k_zero_u32, dim3(1), dim3(128), 0, s, (uint32_t *)p, kCRTok + 1);
         MH_TRY(hip_check(hipGetLastError(), "counter clear"));
     }
+    *cnt = (unsigned *)p;
+    return MH_OK;
+}
+
+int launch_combine_route(const DevLayer &L, float *x, const float *ye, const float *wprev, int n, float *xb,
+                         float *rl, int32_t *sel, float *w, uint32_t *usage, const GroupTab &tab, int unfilled,
+                         unsigned *cnt, hipStream_t s) {
+    if (!combine_route_ok(L, n)) return MH_E_UNSUPPORTED;
     CombineRouteArgs A;
     A.x = x;
     A.ye = ye;
@@ -912,7 +926,7 @@ int launch_combine_route(const DevLayer &L, float *x, const float *ye, const flo
     A.w = w;
     A.usage = usage;
     A.tab = tab;
-    A.cnt = (unsigned *)cp;
+    A.cnt = cnt;
     const dim3 grid((unsigned)n, (unsigned)((L.n_experts + kCRRows - 1) / kCRRows));
 #define CR_LAUNCH(DT, PER) MH_LAUNCH("combine_route", (k_combine_route<DT, PER>), grid, dim3(1024), 0, s, A)
     if (L.router.dt == MH_DT_Q8R) {
@@ -993,42 +1007,51 @@ int layer_bufs(const DevLayer &L, int n, LayerBufs *b, bool need_h = true) {
     MH_TRY(scratch(S_W, (uint64_t)n * L.top_k * 4, &p));
     b->w = (float *)p;
     b->tab = {};
-    const uint64_t N = (uint64_t)n * L.top_k;
-    if (scratch(S_ORD, group_tab_ints(N) * 4, &p) == MH_OK) b->tab = group_tab(p, N);
-    else clear_error();   // over the memory limit: the kernels that walk sel as it is
     return MH_OK;
 }
 
-// Router (rmsnorm, logits, top-k) for n tokens into b->xb / b->sel / b->w
-// (and the table of groups when `tab` is not null).
+// The table of groups of n tokens' assignments, for the paths that use one.
+// Its memory is taken after all else that the call needs, and a call that
+// has none left runs without it (null order); any other failure is the call's.
+int table_buf(const DevLayer &L, int n, LayerBufs *b) {
+    void *p;
+    const uint64_t N = (uint64_t)n * L.top_k;
+    const int rc = scratch(S_ORD, group_tab_ints(N) * 4, &p);
+    if (rc == MH_OK) b->tab = group_tab(p, N);
+    else if (rc == MH_E_NOMEM) clear_error();
+    return rc == MH_E_NOMEM ? MH_OK : rc;
+}
+
+// Router (rmsnorm, logits, top-k) for n tokens into b.xb / b.sel / b.w, and
+// into b.tab where a table is wanted and there is memory for one.
 // x null: b.xb already holds rmsnorm(x) of this layer (k_combine_norm).
-int run_router(const DevLayer &L, const float *x, int n, int unfilled, const LayerBufs &b, uint32_t *usage,
-               const GroupTab *tab, hipStream_t s) {
+int run_router(const DevLayer &L, const float *x, int n, int unfilled, LayerBufs &b, uint32_t *usage, bool want_tab,
+               hipStream_t s) {
     if (x) MH_TRY(launch_rmsnorm(x, L.mlp_norm, b.xb, L.hidden, L.norm_eps, n, s));
     MH_TRY(launch_gemv(L.router, b.xb, b.rl, n, s));
-    return launch_topk(b.rl, L.router_b, n, L.n_experts, L.top_k, L.router_norm, unfilled, b.sel, b.w, usage, tab,
-                       s);
+    if (want_tab) MH_TRY(table_buf(L, n, &b));
+    return launch_topk(b.rl, L.router_b, n, L.n_experts, L.top_k, L.router_norm, unfilled, b.sel, b.w, usage,
+                       b.order() ? &b.tab : nullptr, s);
 }
 
 // Two tokens or more through MXFP4 experts take the expert-grouped matrix-core
 // kernels (each routed expert read once for its tokens); the BATCH_GEMV
 // switch, or a layer they cannot run, keeps the per-assignment GEMVs.
-bool decode_grouped(const DevLayer &L, int n, const LayerBufs &b) {
-    return b.order() && !sw(SW_BATCH_GEMV) && !sw(SW_NO_MFMA) && grouped_ok(L, n);
-}
+bool decode_grouped(const DevLayer &L, int n) { return !sw(SW_BATCH_GEMV) && !sw(SW_NO_MFMA) && grouped_ok(L, n); }
+// (the GEMVs walk the assignments by expert up to 16 tokens, where the top-k's
+// own block writes the order)
+bool decode_table(const DevLayer &L, int n) { return n <= 16 || decode_grouped(L, n); }
 
 // exact: the layer's scales are known to be carried by f16 (a stack's plan
 // scanned them). have_xb: b.xb holds this layer's normed input already; next:
 // the next layer, whose RMSNorm is fused into this layer's combine (or null).
-int run_decode_layer(const DevLayer &L, float *x, int n, const LayerBufs &b, uint32_t *usage, hipStream_t s,
+int run_decode_layer(const DevLayer &L, float *x, int n, LayerBufs b, uint32_t *usage, hipStream_t s,
                      bool exact = false, bool have_xb = false, const DevLayer *next = nullptr) {
-    const bool grouped = decode_grouped(L, n, b);
-    const bool tab = b.order() && (grouped || n <= 16);   // the GEMVs' walk by expert: up to 16 tokens, in the top-k
-    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, tab ? &b.tab : nullptr, s));
-    if (grouped)
+    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, decode_table(L, n), s));
+    if (b.order() && decode_grouped(L, n))
         MH_TRY(launch_grouped(L, n, b.tab, b.xb, b.h, b.ye, exact, s));
     else
-        MH_TRY(launch_experts(L, n * L.top_k, b.sel, tab ? b.order() : nullptr, b.xb, b.h, b.ye, s));
+        MH_TRY(launch_experts(L, n * L.top_k, b.sel, b.order(), b.xb, b.h, b.ye, s));
     if (next) {
         MH_LAUNCH("combine_norm", k_combine_norm, dim3((unsigned)n), dim3(1024), 0, s, x, b.ye, b.w, L.hidden, L.top_k,
                   next->mlp_norm, next->norm_eps, b.xb);
@@ -1056,21 +1079,25 @@ bool prefill_gemm(const DevLayer &L, int n) {
 // from two tokens on, as a decode step of as many does (their terms are f32's
 // own accuracy); the per-assignment GEMVs run the rest: one token, other
 // types and shapes, NO_MFMA.
-bool prefill_grouped(const DevLayer &L, int n, const LayerBufs &b) {
-    return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && b.order() && grouped_ok(L, n);
+bool prefill_grouped(const DevLayer &L, int n) {
+    return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && grouped_ok(L, n);
 }
 
-// have_tab: b.tab holds the groups of sel already; xb null: the records of the
-// normed inputs are written already (prefill_gemm only).
+// b.tab: the groups of sel, or null where the router has not written them;
+// xb null: the records of the normed inputs are written already (prefill_gemm
+// only).
 int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *sel, const float *w, float *x,
-                     const LayerBufs &b, bool have_tab, hipStream_t s) {
+                     LayerBufs b, hipStream_t s) {
     if (prefill_gemm(L, n)) {
         MH_TRY(run_expert_major_mfma(L, n, xb, sel, b.ye, s));
-    } else if (prefill_grouped(L, n, b)) {
-        if (!have_tab) MH_TRY(launch_groups(sel, n * L.top_k, L.n_experts, b.tab, s));
-        MH_TRY(launch_grouped(L, n, b.tab, xb, b.h, b.ye, false, s));
     } else {
-        MH_TRY(launch_experts(L, n * L.top_k, sel, have_tab ? b.order() : nullptr, xb, b.h, b.ye, s));
+        const bool grouped = prefill_grouped(L, n);
+        if (grouped && !b.order()) {
+            MH_TRY(table_buf(L, n, &b));
+            if (b.order()) MH_TRY(launch_groups(sel, n * L.top_k, L.n_experts, b.tab, s));
+        }
+        if (grouped && b.order()) MH_TRY(launch_grouped(L, n, b.tab, xb, b.h, b.ye, false, s));
+        else MH_TRY(launch_experts(L, n * L.top_k, sel, b.order(), xb, b.h, b.ye, s));
     }
     if (L.hidden % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)b.ye % 16 == 0)
         MH_LAUNCH("combine_prefill", k_combine_prefill4, dim3((unsigned)((L.hidden / 4 + 255) / 256), (unsigned)n),
@@ -1085,12 +1112,13 @@ int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *s
 // per token) and the expert-major block on its choice. Up to kCRTok tokens
 // are routed in one launch, which also leaves the table of groups, more in
 // one that also leaves the matrix product's records.
-int run_prefill(const DevLayer &L, float *x, int n, const LayerBufs &b, hipStream_t s) {
-    bool have_tab = false;
+int run_prefill(const DevLayer &L, float *x, int n, LayerBufs b, hipStream_t s) {
     const float *xb = b.xb;
-    if (b.order() && !sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n)) {
-        MH_TRY(launch_combine_route(L, x, nullptr, nullptr, n, b.xb, b.rl, b.sel, b.w, nullptr, b.tab, 0, s));
-        have_tab = true;
+    unsigned *cnt = nullptr;
+    if (!sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n)) MH_TRY(route_counters(&cnt, s));
+    if (cnt) {
+        if (prefill_grouped(L, n)) MH_TRY(table_buf(L, n, &b));
+        MH_TRY(launch_combine_route(L, x, nullptr, nullptr, n, b.xb, b.rl, b.sel, b.w, nullptr, b.tab, 0, cnt, s));
     } else if (n > kCRTok && !sw(SW_SPLIT_ROUTE) && route_tokens_ok(L)) {
         uint8_t *rec = nullptr, *hq;
         if (prefill_gemm(L, n)) {
@@ -1099,10 +1127,9 @@ int run_prefill(const DevLayer &L, float *x, int n, const LayerBufs &b, hipStrea
         }
         MH_TRY(launch_route_tokens(L, x, n, rec ? nullptr : b.xb, rec, b.sel, b.w, 0, s));
     } else {
-        have_tab = prefill_grouped(L, n, b);
-        MH_TRY(run_router(L, x, n, 0, b, nullptr, have_tab ? &b.tab : nullptr, s));
+        MH_TRY(run_router(L, x, n, 0, b, nullptr, prefill_grouped(L, n), s));
     }
-    return run_expert_major(L, n, xb, b.sel, b.w, x, b, have_tab, s);
+    return run_expert_major(L, n, xb, b.sel, b.w, x, b, s);
 }
 
 int check_tokens(int n, const char *what) {
@@ -1348,7 +1375,7 @@ int mh_expert_major_dev(const mh_moe_layer *Lh, int n, const float *xb, const in
     MH_TRY(resolve_dev(x, (uint64_t)n * L.hidden * 4, "mh_expert_major_dev x"));
     LayerBufs b;
     MH_TRY(layer_bufs(L, n, &b, !prefill_gemm(L, n)));
-    return run_expert_major(L, n, xb, sel, w, x, b, false, stream());
+    return run_expert_major(L, n, xb, sel, w, x, b, stream());
 }
 
 int mh_moe_prefill_dev(const mh_moe_layer *Lh, int n, float *x, int32_t *sel, float *w) {
@@ -1442,9 +1469,14 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
     LayerBufs b;
     MH_TRY(layer_bufs(L0, batch, &b));
     const bool exact = step_plan_few(st->plan);
-    bool fuse = b.order() && !sw(SW_SPLIT_ROUTE);
+    bool fuse = !sw(SW_SPLIT_ROUTE);
     for (int l = 0; l < nl && fuse; l++) fuse = combine_route_ok(st->layers[(size_t)l], batch);
-    if (fuse) {
+    unsigned *cnt = nullptr;
+    if (fuse) MH_TRY(route_counters(&cnt, s));
+    if (cnt) {
+        bool want_tab = false;
+        for (int l = 0; l < nl; l++) want_tab |= decode_table(st->layers[(size_t)l], batch);
+        if (want_tab) MH_TRY(table_buf(L0, batch, &b));
         // each layer boundary (the previous layer's combine, this layer's
         // norm, router and top-k) in one launch; the sel / w of a layer in
         // the caller's rows or, without them, in place in the scratch (a
@@ -1454,16 +1486,16 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
         auto lw = [&](int l) { return w ? w + (size_t)l * batch * k : b.w; };
         auto luse = [&](int l) { return usage ? usage + (size_t)l * L0.n_experts : nullptr; };
         MH_TRY(launch_combine_route(L0, x, nullptr, nullptr, batch, b.xb, b.rl, lsel(0), lw(0), luse(0), b.tab, -1,
-                                    s));
+                                    cnt, s));
         for (int l = 0; l < nl; l++) {
             const DevLayer &L = st->layers[(size_t)l];
-            if (decode_grouped(L, batch, b))
+            if (b.order() && decode_grouped(L, batch))
                 MH_TRY(launch_grouped(L, batch, b.tab, b.xb, b.h, b.ye, exact, s));
             else
                 MH_TRY(launch_experts(L, batch * k, lsel(l), b.order(), b.xb, b.h, b.ye, s));
             if (l + 1 < nl) {
                 MH_TRY(launch_combine_route(st->layers[(size_t)l + 1], x, b.ye, lw(l), batch, b.xb, b.rl, lsel(l + 1),
-                                            lw(l + 1), luse(l + 1), b.tab, -1, s));
+                                            lw(l + 1), luse(l + 1), b.tab, -1, cnt, s));
             } else {
                 MH_LAUNCH("combine_decode", k_combine_decode, dim3((unsigned)((L.hidden + 255) / 256), (unsigned)batch),
                           dim3(256), 0, s, x, b.ye, lw(l), L.hidden, L.top_k);
@@ -1504,7 +1536,7 @@ int mh_stack_apply_dev(mh_stack *st, int layer, const float *xb, const int32_t *
     }
     LayerBufs b;
     MH_TRY(layer_bufs(L, 1, &b));
-    return run_expert_major(L, 1, xb, sel, w, x, b, false, s);
+    return run_expert_major(L, 1, xb, sel, w, x, b, s);
 }
 
 int mh_stack_destroy(mh_stack *st) {

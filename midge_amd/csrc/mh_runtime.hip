@@ -327,6 +327,16 @@ int async_flag(AsyncFlag id, const char *msg, unsigned **dev) {
     return MH_OK;
 }
 
+// Gives a slot's memory back (after the work that may use it).
+static int drop_scratch(Scratch slot) {
+    MH_HIP(hipStreamSynchronize(g.cur));
+    MH_HIP(hipFree(g.scratch[slot]));
+    g.allocated -= g.scratch_bytes[slot];
+    g.scratch[slot] = nullptr;
+    g.scratch_bytes[slot] = 0;
+    return MH_OK;
+}
+
 int scratch(Scratch slot, uint64_t bytes, void **p, bool *fresh) {
     if (fresh) *fresh = false;
     if (bytes <= g.scratch_bytes[slot] && g.scratch[slot]) {
@@ -334,15 +344,18 @@ int scratch(Scratch slot, uint64_t bytes, void **p, bool *fresh) {
         return MH_OK;
     }
     if (fresh) *fresh = true;
-    if (g.scratch[slot]) {
-        MH_HIP(hipStreamSynchronize(g.cur));
-        MH_HIP(hipFree(g.scratch[slot]));
-        g.allocated -= g.scratch_bytes[slot];
-        g.scratch[slot] = nullptr;
-        g.scratch_bytes[slot] = 0;
-    }
+    if (g.scratch[slot]) MH_TRY(drop_scratch(slot));
     uint64_t want = bytes < 4096 ? 4096 : bytes + bytes / 4;
-    MH_TRY(dev_malloc(&g.scratch[slot], want, "scratch"));
+    int rc = dev_malloc(&g.scratch[slot], want, "scratch");
+    // the table of groups and the one-launch router's counters are what calls
+    // can do without, and they take them last: an earlier call's give way
+    for (Scratch o : {S_ORD, S_CROUTE})
+        if (rc == MH_E_NOMEM && slot != S_ORD && slot != S_CROUTE && g.scratch[o]) {
+            MH_TRY(drop_scratch(o));
+            clear_error();
+            rc = dev_malloc(&g.scratch[slot], want, "scratch");
+        }
+    MH_TRY(rc);
     g.scratch_bytes[slot] = want;
     *p = g.scratch[slot];
     return MH_OK;
