@@ -94,11 +94,14 @@ int mh_sync(void);
 /* Path switches for comparisons (tests, benchmarks), all off by default.
  * mh_init reads each from the environment once (MIDGE_HIP_<name> set and not
  * "0"); this call changes one at run time: "NO_MFMA" (no matrix-core
- * kernels in the batched int8 GEMV, the prefill and the decode step),
+ * kernels in the batched int8 GEMV, the prefill and decode steps),
  * "NO_FUSED" (stack decode as per-layer launches), "ATTN_SPLIT" (attention
  * as four launches), "COOP" (the one-launch decode step launched
  * cooperatively), "Q8_NO_ROWS" (long batched int8 GEMVs on the
- * register-operand kernel). MH_E_ARG for an unknown name. No counterpart in
+ * register-operand kernel), "BATCH_GEMV" (decode steps of several tokens on
+ * the per-assignment GEMVs), "GROUPED" (decode steps and short prefills of
+ * several tokens on the expert-grouped kernels wherever they can run),
+ * "SPLIT_ROUTE" (a layer's router as three launches). MH_E_ARG for an unknown name. No counterpart in
  * the reference: its only comparable knob is MIDGE_NO_SIMD, read once at
  * start-up (engine/mkern.h:75-93). */
 int mh_set_switch(const char *name, int on);

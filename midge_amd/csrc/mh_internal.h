@@ -78,10 +78,13 @@ int async_flag(AsyncFlag id, const char *msg, unsigned **dev);
 //   Q8_NO_ROWS  long batched int8 GEMVs on the register-operand kernel
 //   BATCH_GEMV  decode steps of several tokens on the per-assignment GEMVs
 //               instead of the expert-grouped matrix-core kernels
+//   GROUPED     decode steps and short prefills of two tokens or more on the
+//               expert-grouped kernels wherever they can run
 //   SPLIT_ROUTE a stack decode's layer boundary (combine, norm, router,
 //               top-k), or a prefill's router, as three launches instead of
 //               k_combine_route or k_route_tokens
-enum Switch { SW_NO_MFMA = 0, SW_NO_FUSED, SW_ATTN_SPLIT, SW_COOP, SW_Q8_NO_ROWS, SW_BATCH_GEMV, SW_SPLIT_ROUTE, SW_COUNT };
+enum Switch { SW_NO_MFMA = 0, SW_NO_FUSED, SW_ATTN_SPLIT, SW_COOP, SW_Q8_NO_ROWS, SW_BATCH_GEMV, SW_SPLIT_ROUTE, SW_GROUPED,
+              SW_COUNT };
 bool sw(Switch s);
 
 // The number of successful mh_init calls so far (never reset): state that a

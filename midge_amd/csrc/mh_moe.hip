@@ -6,6 +6,7 @@
 //   mh_topk_dev                 route_topk() selection, engine/midge.c:410-433
 //   mh_expert_major_dev         expert-major loop + expert_apply, midge.c:595-611, 437-467
 //   mh_stack_*                  forward()'s layer loop, MoE half, midge.c:557-560
+#include <cmath>
 #include <vector>
 
 #include "mh_fp6.cuh"
@@ -782,6 +783,22 @@ k_combine_prefill4(float *__restrict__ x, const float *__restrict__ ye, const in
     *(float4 *)(x + (size_t)t * H + r) = acc;
 }
 
+// The grid of the per-assignment GEMVs: rpb of an assignment's `rows` rows to a
+// block (a multiple of step), so that the blocks of all A are two to a CU.
+struct RowSplit {
+    int64_t rpb, nblk;
+};
+RowSplit expert_rows(int64_t rows, int A, int64_t step, int64_t most) {
+    const int64_t target = (int64_t)device_cus() * 2;
+    const int64_t per = (rows * A + target - 1) / target;   // rows per block
+    int64_t rpb = ((per + step - 1) / step) * step;
+    if (rpb < step) rpb = step;
+    if (rpb > most) rpb = most;
+    return {rpb, (rows + rpb - 1) / rpb};
+}
+RowSplit gu_rows(int64_t ffn, int A, int ns) { return expert_rows(ffn, A, (ns + 1) / 2, 2048); }   // pairs of rows
+RowSplit down_rows(int64_t hidden, int A, int ns) { return expert_rows(hidden, A, ns, 4096); }
+
 template <int DT>
 int launch_experts_t(const DevLayer &L, int A, const int32_t *sel, const int32_t *order, const float *xb, float *h,
                      float *ye, hipStream_t s) {
@@ -797,17 +814,11 @@ int launch_experts_t(const DevLayer &L, int A, const int32_t *sel, const int32_t
     ea.alpha = L.alpha;
     ea.limit = L.limit;
     ea.act_plain = L.act_plain;
-    const int64_t target = (int64_t)device_cus() * 2;
     {   // gate/up: 2 * ffn flat rows per assignment
         const int C = (int)(L.hidden / CE);
         int ns, nt;
         gemv_shape(C, &ns, &nt);
-        int64_t per = (L.ffn * A + target - 1) / target;   // rows per block
-        int64_t step = (ns + 1) / 2;
-        int64_t rpb = ((per + step - 1) / step) * step;
-        if (rpb < step) rpb = step;
-        if (rpb > 2048) rpb = 2048;
-        const int64_t nblk = (L.ffn + rpb - 1) / rpb;
+        const auto [rpb, nblk] = gu_rows(L.ffn, A, ns);
         const size_t lds = ((size_t)2 * rpb + gemv_lds_floats(ns, C)) * sizeof(float);
         MH_LAUNCH("expert_gu", k_expert_gu<DT>, dim3((unsigned)nblk, (unsigned)A), dim3(nt), lds, s, ea, sel, order, xb,
                            h, ns, (int)rpb);
@@ -817,11 +828,7 @@ int launch_experts_t(const DevLayer &L, int A, const int32_t *sel, const int32_t
         const int C = (int)(L.ffn / CE);
         int ns, nt;
         gemv_shape(C, &ns, &nt);
-        int64_t per = (L.hidden * A + target - 1) / target;
-        int64_t rpb = ((per + ns - 1) / ns) * ns;
-        if (rpb < ns) rpb = ns;
-        if (rpb > 4096) rpb = 4096;
-        const int64_t nblk = (L.hidden + rpb - 1) / rpb;
+        const auto [rpb, nblk] = down_rows(L.hidden, A, ns);
         const size_t lds = ((size_t)rpb + gemv_lds_floats(ns, C)) * sizeof(float);
         MH_LAUNCH("expert_down", k_expert_down<DT>, dim3((unsigned)nblk, (unsigned)A), dim3(nt), lds, s, ea, sel, order, h,
                            ye, ns, (int)rpb);
@@ -1034,21 +1041,51 @@ int run_router(const DevLayer &L, const float *x, int n, int unfilled, LayerBufs
                        b.order() ? &b.tab : nullptr, s);
 }
 
-// Two tokens or more through MXFP4 experts take the expert-grouped matrix-core
-// kernels (each routed expert read once for its tokens); the BATCH_GEMV
-// switch, or a layer they cannot run, keeps the per-assignment GEMVs.
-bool decode_grouped(const DevLayer &L, int n) { return !sw(SW_BATCH_GEMV) && !sw(SW_NO_MFMA) && grouped_ok(L, n); }
+// Whether the expert-grouped kernels (each routed expert read once) are the
+// faster ones for n tokens. The GEMVs take as long as the bytes of all
+// assignments need, or half as long again where their blocks leave a third
+// on some CUs (17-31 assignments of a 2880-wide layer: 97-111 us, 32: 95); the
+// grouped kernels stream the expected number of different experts at 1 / 1.1 of
+// that rate and cost about 50 MB more to start (staging, the table).
+// Measured us, GEMVs / grouped, by whole prefills of layers that no cache
+// holds (128 experts, top-4): 2880 wide 4 tokens 65 / 70, 6 106 / 88, 16 157 /
+// 142, 64 613 / 280; 2048 x 1536 8 tokens 53 / 58, 10 74 / 62, 16 73 / 80, 24
+// 133 / 93; 1024 x 768 16 tokens 43 / 45, 24 58 / 50, 64 90 / 77; 256 x 192 24
+// 36 / 36, 64 42 / 45. Of 1500 calls (prefills, moe and stack decodes of 2-192
+// tokens, 32-128 experts, top-2 to top-8) the side taken is on average 0.9%
+// slower than the better one, at most 15%.
+bool grouped_pays(const DevLayer &L, int n) {
+    const int N = n * L.top_k, C = (int)(L.hidden / 32), Cd = (int)(L.ffn / 32);
+    int ns, nt;
+    gemv_shape(C, &ns, &nt);
+    const RowSplit gu = gu_rows(L.ffn, N, ns);
+    gemv_shape(Cd, &ns, &nt);
+    const RowSplit dn = down_rows(L.hidden, N, ns);
+    const int64_t cus = device_cus();
+    auto whole = [&](const RowSplit &r) { return (double)((r.nblk * N + cus - 1) / cus * cus) * (double)r.rpb; };
+    const double gemv = 18.0 * (2.0 * whole(gu) * C + whole(dn) * Cd);   // 16 bytes of codes and a scale a chunk
+    const double used = L.n_experts * (1.0 - std::pow(1.0 - (double)L.top_k / L.n_experts, n));
+    return gemv - 1.1 * used * (double)L.expert_stride > 50e6;
+}
+
+// Which decode steps take the expert-grouped kernels: those of a scanned stack
+// (exact) up to 16 tokens and 64 assignments, others where they pay. The GROUPED
+// switch takes them wherever they can run, BATCH_GEMV nowhere.
+bool decode_grouped(const DevLayer &L, int n, bool exact) {
+    if (sw(SW_BATCH_GEMV) || sw(SW_NO_MFMA) || !grouped_ok(L, n)) return false;
+    return sw(SW_GROUPED) || (exact && n <= 16 && n * L.top_k <= 64) || grouped_pays(L, n);
+}
 // (the GEMVs walk the assignments by expert up to 16 tokens, where the top-k's
 // own block writes the order)
-bool decode_table(const DevLayer &L, int n) { return n <= 16 || decode_grouped(L, n); }
+bool decode_table(const DevLayer &L, int n, bool exact) { return n <= 16 || decode_grouped(L, n, exact); }
 
 // exact: the layer's scales are known to be carried by f16 (a stack's plan
 // scanned them). have_xb: b.xb holds this layer's normed input already; next:
 // the next layer, whose RMSNorm is fused into this layer's combine (or null).
 int run_decode_layer(const DevLayer &L, float *x, int n, LayerBufs b, uint32_t *usage, hipStream_t s,
                      bool exact = false, bool have_xb = false, const DevLayer *next = nullptr) {
-    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, decode_table(L, n), s));
-    if (b.order() && decode_grouped(L, n))
+    MH_TRY(run_router(L, have_xb ? nullptr : x, n, -1, b, usage, decode_table(L, n, exact), s));
+    if (b.order() && decode_grouped(L, n, exact))
         MH_TRY(launch_grouped(L, n, b.tab, b.xb, b.h, b.ye, exact, s));
     else
         MH_TRY(launch_experts(L, n * L.top_k, b.sel, b.order(), b.xb, b.h, b.ye, s));
@@ -1076,11 +1113,10 @@ bool prefill_gemm(const DevLayer &L, int n) {
 }
 
 // A prefill of fewer tokens per expert takes the expert-grouped f16 kernels
-// from two tokens on, as a decode step of as many does (their terms are f32's
-// own accuracy); the per-assignment GEMVs run the rest: one token, other
-// types and shapes, NO_MFMA.
+// where they pay, as a decode step of as many does; the per-assignment GEMVs
+// run the rest: few assignments, other types and shapes, NO_MFMA.
 bool prefill_grouped(const DevLayer &L, int n) {
-    return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && grouped_ok(L, n);
+    return !prefill_gemm(L, n) && !sw(SW_NO_MFMA) && grouped_ok(L, n) && (sw(SW_GROUPED) || grouped_pays(L, n));
 }
 
 // b.tab: the groups of sel, or null where the router has not written them;
@@ -1475,7 +1511,7 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
     if (fuse) MH_TRY(route_counters(&cnt, s));
     if (cnt) {
         bool want_tab = false;
-        for (int l = 0; l < nl; l++) want_tab |= decode_table(st->layers[(size_t)l], batch);
+        for (int l = 0; l < nl; l++) want_tab |= decode_table(st->layers[(size_t)l], batch, exact);
         if (want_tab) MH_TRY(table_buf(L0, batch, &b));
         // each layer boundary (the previous layer's combine, this layer's
         // norm, router and top-k) in one launch; the sel / w of a layer in
@@ -1489,7 +1525,7 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
                                     cnt, s));
         for (int l = 0; l < nl; l++) {
             const DevLayer &L = st->layers[(size_t)l];
-            if (b.order() && decode_grouped(L, batch))
+            if (b.order() && decode_grouped(L, batch, exact))
                 MH_TRY(launch_grouped(L, batch, b.tab, b.xb, b.h, b.ye, exact, s));
             else
                 MH_TRY(launch_experts(L, batch * k, lsel(l), b.order(), b.xb, b.h, b.ye, s));

@@ -1,13 +1,13 @@
 """The expert-grouped f16 kernels past 16 tokens and in short prefills: against
 the per-assignment GEMVs on the same weights, at the edges of their ranges
 (groups of 4, one-launch routing up to 64 tokens, partly filled units of 8
-tiles) and with scales that f16 terms cannot carry."""
+tiles) and with scales that f16 terms cannot carry; and which calls take them."""
 import numpy as np
 import pytest
 
 from conftest import rel_l2, say
-from midge_amd import DevBuf, synth
-from midge_amd.moe import MoELayer, Stack, expert_major_dev, moe_prefill
+from midge_amd import DevBuf, device, synth
+from midge_amd.moe import MoELayer, Stack, expert_major_dev, moe_dev, moe_prefill, moe_prefill_dev
 from midge_amd.synth import Keys, MoEShape
 from oracle import pyoracle as po
 
@@ -45,6 +45,7 @@ def make(shape, seed, scales="plain", bias=None):
 ], ids=lambda v: v if isinstance(v, (int, str)) else f"{v.hidden}x{v.ffn}e{v.n_experts}")
 def test_short_prefill(mh, path_switch, shape, n, scales):
     say(f"short prefill {shape.hidden}x{shape.ffn} E={shape.n_experts} n={n} scales={scales}")
+    path_switch("GROUPED")
     keys, arrays, lay = make(shape, 11, scales)
     X = synth.host_x(shape, keys, n, step=2)
     xg, selg, wg = moe_prefill(lay, X)
@@ -70,6 +71,7 @@ def test_stack_many_tokens(mh, path_switch, shape, n, unfilled):
         b[[2, 11]] = 0.0
         return b
 
+    path_switch("GROUPED")
     keys, arrays, lay = make(shape, 12, bias=bias if unfilled else None)
     X, k = synth.host_x(shape, keys, n, step=1), shape.top_k
     st = Stack([lay], max_batch=n)
@@ -99,6 +101,7 @@ def test_given_routing_with_unroutable_slots(mh, path_switch):
     """mh_expert_major_dev takes any selection: slots outside [0, E) add nothing."""
     shape, n = MID, 40
     say("expert major, unroutable slots")
+    path_switch("GROUPED")
     keys, arrays, lay = make(shape, 13)
     X = synth.host_x(shape, keys, n, step=4)
     rng = np.random.default_rng(5)
@@ -118,3 +121,49 @@ def test_given_routing_with_unroutable_slots(mh, path_switch):
     assert np.array_equal(out[0][7], X[7])
     for t in range(n):
         assert rel_l2(out[0][t], out[1][t]) < TOL, t
+
+
+@pytest.mark.parametrize("kind,n,grouped", [("prefill", 2, False), ("prefill", 8, False), ("prefill", 63, True),
+                                            ("experts", 8, False), ("experts", 48, True), ("moe", 2, False),
+                                            ("moe", 8, False), ("moe", 64, True), ("stack", 16, True), ("stack", 17, True),
+                                            ("stack", 64, True)])
+def test_route(mh, path_switch, kind, n, grouped):
+    """Few assignments of a small layer run on the GEMVs, many on the grouped
+    kernels (a scanned stack's up to 64 assignments in any case); where the
+    GEMVs run, the result is theirs bit for bit."""
+    shape, k = MoEShape(hidden=1024, ffn=768, n_experts=32, top_k=4), 4
+    say(f"route {kind} n={n}")
+    keys, arrays, lay = make(shape, 14)
+    X = synth.host_x(shape, keys, n, step=1)
+    rng = np.random.default_rng(n)
+    sel = np.argsort(rng.random((n, shape.n_experts)), axis=1)[:, :k].astype(np.int32)
+    w = np.full((n, k), 0.25, np.float32)
+    st = Stack([lay], max_batch=64) if kind == "stack" else None
+    out = []
+    for gemv in (False, True):
+        path_switch("NO_MFMA" if kind in ("prefill", "experts") else "BATCH_GEMV", gemv)
+        xd, xb, sd, wd = (DevBuf.from_array(a) for a in (X, X, sel, w))
+        device.profile_enable()
+        device.profile_reset()
+        if kind == "prefill":
+            moe_prefill_dev(lay, xd, n, sd, wd)
+        elif kind == "experts":
+            expert_major_dev(lay, n, xb, sd, wd, xd)
+        elif kind == "moe":
+            moe_dev(lay, xd, n, sd, wd)
+        else:
+            st.decode(xd, n, sd, wd)
+        mh.sync()
+        ran = device.profile_query("grouped_gu")[1], device.profile_query("expert_gu")[1]
+        device.profile_enable(False)
+        assert ran == ((0, 1) if gemv or not grouped else (1, 0))
+        out.append(xd.download(np.float32, X.shape))
+        for d in (xd, xb, sd, wd):
+            d.free()
+    if st:
+        st.destroy()
+    lay.release()
+    if grouped:
+        assert max(rel_l2(a, b) for a, b in zip(*out)) < TOL
+    else:
+        assert np.array_equal(*out)
