@@ -6,6 +6,7 @@
 //   mh_topk_dev                 route_topk() selection, engine/midge.c:410-433
 //   mh_expert_major_dev         expert-major loop + expert_apply, midge.c:595-611, 437-467
 //   mh_stack_*                  forward()'s layer loop, MoE half, midge.c:557-560
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -888,6 +889,17 @@ bool combine_route_ok(const DevLayer &L, int n) {
            (uint64_t)L.n_experts * (uint64_t)L.hidden * (L.router.dt == MH_DT_Q8R ? 1u : 4u) < (1ull << 32);
 }
 
+// Whether it is the faster router there: its blocks (16 experts of a token
+// each) form the token's input again, so past two to a CU it loses to the three
+// launches unless the rows are long. Whole prefills with experts of 64, one
+// launch / three, us: 64 tokens, 128 experts, hidden 256 34 / 33, 1024 39 / 39,
+// 2880 47 / 56; 256 experts 43 / 34, 49 / 44, 60 / 71; 1024 experts 91 / 45, 108
+// / 77, 141 / 154 (2048: 122 / 114); 16 tokens, 1024 experts 49 / 38, 50 / 44,
+// 61 / 69.
+bool combine_route_pays(const DevLayer &L, int n) {
+    return (int64_t)n * ((L.n_experts + kCRRows - 1) / kCRRows) <= 2 * (int64_t)device_cus() || L.hidden > 2048;
+}
+
 // Its arrival counters; null where the memory cap leaves none (the caller
 // routes in separate launches, which need none).
 int route_counters(unsigned **cnt, hipStream_t s) {
@@ -954,6 +966,19 @@ int launch_combine_route(const DevLayer &L, float *x, const float *ye, const flo
 bool route_tokens_ok(const DevLayer &L) {
     return L.router.dt == MH_DT_Q8R && L.hidden % 32 == 0 && L.hidden <= kCRMaxH && L.n_experts <= kMaxExperts &&
            (uintptr_t)L.router.data % 16 == 0;
+}
+
+// Whether it is the faster router there: a wave walks every expert with room
+// for rows of kCRMaxH, whatever their length, so many experts of short rows are
+// quicker in separate launches. Whole prefills with experts of 64, one launch /
+// three, us: hidden 64 2047 tokens, 64 experts 63 / 65, 128 88 / 66, 1024 497 /
+// 172; hidden 256, 128 experts 98 / 85, 1024 581 / 394; hidden 512, 128 experts
+// 65 tokens 38 / 37, 200 40 / 43, 2047 98 / 124, 256 experts 96 tokens 47 / 42, 200
+// 48 / 51, 1024 experts 96 / 98, 2047 547 / 706; hidden 1024, 128 experts 65
+// tokens 38 / 41, 1024 experts 65 94 / 79, 96 98 / 98, 200 111 / 164.
+bool route_tokens_pays(const DevLayer &L, int n) {
+    return L.n_experts <= 64 ||
+           (L.hidden >= 512 && (int64_t)n * L.hidden >= std::min<int64_t>(400 * (int64_t)L.n_experts, 100000));
 }
 
 int launch_route_tokens(const DevLayer &L, const float *x, int n, float *xb, uint8_t *rec, int32_t *sel, float *w,
@@ -1151,11 +1176,11 @@ int run_expert_major(const DevLayer &L, int n, const float *xb, const int32_t *s
 int run_prefill(const DevLayer &L, float *x, int n, LayerBufs b, hipStream_t s) {
     const float *xb = b.xb;
     unsigned *cnt = nullptr;
-    if (!sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n)) MH_TRY(route_counters(&cnt, s));
+    if (!sw(SW_SPLIT_ROUTE) && combine_route_ok(L, n) && combine_route_pays(L, n)) MH_TRY(route_counters(&cnt, s));
     if (cnt) {
         if (prefill_grouped(L, n)) MH_TRY(table_buf(L, n, &b));
         MH_TRY(launch_combine_route(L, x, nullptr, nullptr, n, b.xb, b.rl, b.sel, b.w, nullptr, b.tab, 0, cnt, s));
-    } else if (n > kCRTok && !sw(SW_SPLIT_ROUTE) && route_tokens_ok(L)) {
+    } else if (n > kCRTok && !sw(SW_SPLIT_ROUTE) && route_tokens_ok(L) && route_tokens_pays(L, n)) {
         uint8_t *rec = nullptr, *hq;
         if (prefill_gemm(L, n)) {
             MH_TRY(prefill_records(L, n, &rec, &hq));
@@ -1506,7 +1531,10 @@ int mh_stack_decode(mh_stack *st, float *x, int batch, int32_t *sel, float *w, u
     MH_TRY(layer_bufs(L0, batch, &b));
     const bool exact = step_plan_few(st->plan);
     bool fuse = !sw(SW_SPLIT_ROUTE);
-    for (int l = 0; l < nl && fuse; l++) fuse = combine_route_ok(st->layers[(size_t)l], batch);
+    for (int l = 0; l < nl && fuse; l++) {
+        const DevLayer &L = st->layers[(size_t)l];
+        fuse = combine_route_ok(L, batch) && (batch <= 16 || combine_route_pays(L, batch));
+    }
     unsigned *cnt = nullptr;
     if (fuse) MH_TRY(route_counters(&cnt, s));
     if (cnt) {
