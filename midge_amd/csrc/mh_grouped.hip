@@ -461,6 +461,12 @@ bool grouped_ok(const DevLayer &L, int n) {
            L.off[2] % 16 == 0 && L.off[5] % 16 == 0 && L.off[8] % 16 == 0;
 }
 
+// What they read of an expert: codes and scales of K steps in whole groups of
+// kPD (past K a repeat of the row's end, as slow as the rest).
+double grouped_bytes(const DevLayer &L) {
+    return 18.0 * 8.0 * (2.0 * L.ffn * grp_nq((int)L.hidden) + (double)L.hidden * grp_nq((int)L.ffn));
+}
+
 // The expert FFN of n tokens (grouped_ok) from the router's table of groups:
 // h (scratch [N][F]) from xb, then ye [N][H]. exact: every scale of the layer
 // is known to be carried by f16 (a stack's plan has looked).

@@ -186,6 +186,7 @@ inline GroupTab group_tab(void *p, uint64_t N) {
 // h from xb, then ye. grouped_ok: the layer and token count fit. exact: every
 // scale of the layer is known to be zero or a power of two in [2^-23, 2^13].
 bool grouped_ok(const DevLayer &L, int n);
+double grouped_bytes(const DevLayer &L);   // of an expert that the kernels read
 int launch_grouped(const DevLayer &L, int n, const GroupTab &tab, const float *xb, float *h, float *ye, bool exact,
                    hipStream_t s);
 // Runs layers [first, first + n_layers) of a plan in one launch; sel, w and

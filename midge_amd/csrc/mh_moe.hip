@@ -1070,15 +1070,17 @@ int run_router(const DevLayer &L, const float *x, int n, int unfilled, LayerBufs
 // faster ones for n tokens. The GEMVs take as long as the bytes of all
 // assignments need, or half as long again where their blocks leave a third
 // on some CUs (17-31 assignments of a 2880-wide layer: 97-111 us, 32: 95); the
-// grouped kernels stream the expected number of different experts at 1 / 1.1 of
-// that rate and cost about 50 MB more to start (staging, the table).
+// grouped kernels stream the expected number of different experts, in whole
+// groups of K steps (grouped_bytes), at about that rate, and cost about 50 MB
+// more to start and 0.2 MB for each group that is staged.
 // Measured us, GEMVs / grouped, by whole prefills of layers that no cache
-// holds (128 experts, top-4): 2880 wide 4 tokens 65 / 70, 6 106 / 88, 16 157 /
-// 142, 64 613 / 280; 2048 x 1536 8 tokens 53 / 58, 10 74 / 62, 16 73 / 80, 24
-// 133 / 93; 1024 x 768 16 tokens 43 / 45, 24 58 / 50, 64 90 / 77; 256 x 192 24
-// 36 / 36, 64 42 / 45. Of 1500 calls (prefills, moe and stack decodes of 2-192
-// tokens, 32-128 experts, top-2 to top-8) the side taken is on average 0.9%
-// slower than the better one, at most 15%.
+// holds (128 experts, top-4): 2880 wide 4 tokens 67 / 71, 6 106 / 90, 16 162 /
+// 143, 64 600 / 282; 2048 x 1536 8 tokens 51 / 58, 10 72 / 63, 16 73 / 80, 24
+// 127 / 93; 1024 x 768 16 tokens 40 / 45, 24 55 / 51, 64 85 / 77; 512 x 2048, 64
+// experts 16 tokens 43 / 53, 24 64 / 61, 48 97 / 73; 2048 x 192, 64 experts 48
+// tokens 64 / 54, 64 62 / 59. Of 3270 calls (prefills, moe and stack decodes of
+// 2-192 tokens, 32-128 experts, top-2 to top-8, ten widths) the side taken is
+// on average 0.4% slower than the better one, at most 15%.
 bool grouped_pays(const DevLayer &L, int n) {
     const int N = n * L.top_k, C = (int)(L.hidden / 32), Cd = (int)(L.ffn / 32);
     int ns, nt;
@@ -1090,7 +1092,8 @@ bool grouped_pays(const DevLayer &L, int n) {
     auto whole = [&](const RowSplit &r) { return (double)((r.nblk * N + cus - 1) / cus * cus) * (double)r.rpb; };
     const double gemv = 18.0 * (2.0 * whole(gu) * C + whole(dn) * Cd);   // 16 bytes of codes and a scale a chunk
     const double used = L.n_experts * (1.0 - std::pow(1.0 - (double)L.top_k / L.n_experts, n));
-    return gemv - 1.1 * used * (double)L.expert_stride > 50e6;
+    const double groups = used + (N - used) / kGroupTok;
+    return gemv > used * grouped_bytes(L) + 50e6 + 0.2e6 * groups;
 }
 
 // Which decode steps take the expert-grouped kernels: those of a scanned stack
