@@ -1103,9 +1103,13 @@ bool decode_grouped(const DevLayer &L, int n, bool exact) {
     if (sw(SW_BATCH_GEMV) || sw(SW_NO_MFMA) || !grouped_ok(L, n)) return false;
     return sw(SW_GROUPED) || (exact && n <= 16 && n * L.top_k <= 64) || grouped_pays(L, n);
 }
-// (the GEMVs walk the assignments by expert up to 16 tokens, where the top-k's
-// own block writes the order)
-bool decode_table(const DevLayer &L, int n, bool exact) { return n <= 16 || decode_grouped(L, n, exact); }
+// Whether the router writes a table: for the grouped kernels, and up to 16
+// tokens, where the top-k's own block does it, for the GEMVs of layers that those
+// cannot run, to walk the assignments by expert (with few assignments it gains
+// less than the 1.2 us that it takes).
+bool decode_table(const DevLayer &L, int n, bool exact) {
+    return decode_grouped(L, n, exact) || (n <= 16 && !grouped_ok(L, n));
+}
 
 // exact: the layer's scales are known to be carried by f16 (a stack's plan
 // scanned them). have_xb: b.xb holds this layer's normed input already; next:
