@@ -1,8 +1,9 @@
 """The long-matrix batched int8 kernel (k_gemm_q8r_rows) against the register-
 operand kernel on the same digits: their int32 sums are exact, so every output
 is the same bit for bit. Sizes at the edges of its column groups (16-column
-tiles, up to 4), K steps (one chunk of 64, odd and even counts) and row tiles
-(a partial last tile, rows not a multiple of 4)."""
+tiles, up to 4), K steps (one chunk of 64, odd and even counts, rows of whole
+4 KB, whose steps go round from a start of each block's own) and row tiles (a
+partial last tile, rows not a multiple of 4)."""
 import numpy as np
 import pytest
 
@@ -15,7 +16,8 @@ LONG = 131072   # rows from which the long tiling fills a 256-CU card
 
 
 @pytest.mark.parametrize("rows,cols,batch", [(LONG, 64, 2), (LONG + 5, 192, 17), (LONG + 20, 128, 33), (LONG + 3, 640, 64),
-                                             (LONG + 48, 320, 65), (LONG + 16, 64, 130), (201088, 2880, 16)])
+                                             (LONG + 48, 320, 65), (LONG + 16, 64, 130), (201088, 2880, 16),
+                                             (LONG, 4096, 3), (LONG + 37, 8192, 20)])
 def test_rows_kernel_bit_identical(mh, path_switch, rows, cols, batch):
     say(f"q8 rows kernel {rows}x{cols} batch={batch}")
     rng = np.random.default_rng(rows + batch)
