@@ -237,7 +237,9 @@ static_assert(kRows == 128, "a block's rows of h are one K step of the down prod
 // alone are 93 us of the 2000-token gate/up. Slower: one persistent block
 // per CU with the steps running across units (157 + 90 and 427 + 263), the
 // same with half the waves a phase behind (167 + 112 and 412 + 288).)
-template <int MODE>
+// WORDS: weights in 4-byte loads, for tables off a 16-byte boundary (2000 tokens
+// of a 32-expert 2880-wide layer 625 us; 614 in 16-byte loads).
+template <int MODE, bool WORDS>
 __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
     constexpr int NM = MODE == 0 ? 2 : 1;   // weight matrices: gate and up, or down
     extern __shared__ __attribute__((aligned(16))) uint8_t glds[];
@@ -272,19 +274,28 @@ __global__ void __launch_bounds__(64 * kWaves, 2) k_moe_gemm(GemmArgs A) {
 #pragma unroll
     for (int mt = 0; mt < NM; ++mt) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < 2; ++q)   // (R is a multiple of 32: a wave's rows are all there or none)
             aoff[mt][q] = (uint32_t)A.off[MODE == 0 ? 3 * mt : 6] +
-                          (uint32_t)min(row0 + kLoad * q + (l >> 2), R - 1) * (uint32_t)(K / 2) + 16u * swz;
+                          (uint32_t)(min(row0, R - 32) + kLoad * q + (WORDS ? l >> 4 : l >> 2)) * (uint32_t)(K / 2) +
+                          (WORDS ? 4u * (l & 3) : 16u * swz);
         soff[mt] = (uint32_t)A.off[MODE == 0 ? 1 + 3 * mt : 7] + 4u * (l & 7);
     }
-    constexpr int kALoads = 2 * NM, kBLoads = 5;
+    constexpr int kALoads = (WORDS ? 8 : 2) * NM, kBLoads = 5;
     auto issue_a = [&](int st, int buf) __attribute__((always_inline)) {
         // (past K: what follows the row, in the expert's blob; the tokens are zero there)
 #pragma unroll
         for (int mt = 0; mt < NM; ++mt)
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
-                dma16(ldsA + (uint32_t)(buf * gemm_a(NM) + (mt * (kRows / kLoad) + 2 * wave + q) * kLdsAT), ex + 64 * st, aoff[mt][q]);
+            for (int q = 0; q < 2; ++q) {
+                const uint32_t d = ldsA + (uint32_t)(buf * gemm_a(NM) + (mt * (kRows / kLoad) + 2 * wave + q) * kLdsAT);
+                if constexpr (WORDS) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j)   // 4 rows' 64 bytes
+                        dma4(d + 256u * j, ex + 64 * st, aoff[mt][q] + 2u * j * (uint32_t)K + 16u * (((l >> 2) & 3) ^ j));
+                } else {
+                    dma16(d, ex + 64 * st, aoff[mt][q]);
+                }
+            }
     };
     // the scales of 4 steps (32 bytes of a row; 8 rows per load instruction:
     // one step's 8 bytes at a time took as many cache requests as the weights)
@@ -552,12 +563,12 @@ int launch_expert_lists(const int32_t *sel, int N, int E, int k, ExpertLists *ou
 // per-assignment GEMVs' f32 arithmetic).
 constexpr int64_t kMfmaMaxH = 3328, kMfmaMaxF = 4608;
 
-// True when the scaled-MFMA path handles this layer (MXFP4 experts in 16-byte
-// chunks, shapes that tile by 64 along K and 32 along rows).
+// True when the scaled-MFMA path handles this layer (MXFP4 experts on a 4-byte
+// boundary, shapes that tile by 64 along K and 32 along rows).
 bool prefill_mfma_ok(const DevLayer &L) {
     if (sw(SW_NO_MFMA)) return false;
     return L.expert_dt == MH_DT_MXFP4 && L.hidden % 64 == 0 && L.ffn % 64 == 0 && L.top_k >= 1 &&
-           L.n_experts <= kPlistMaxE && L.hidden <= kMfmaMaxH && L.ffn <= kMfmaMaxF && (uintptr_t)L.experts % 16 == 0;
+           L.n_experts <= kPlistMaxE && L.hidden <= kMfmaMaxH && L.ffn <= kMfmaMaxF && (uintptr_t)L.experts % 4 == 0;
 }
 
 // The records of n tokens' x, then of their h (S_Q scratch).
@@ -581,8 +592,10 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
     if (!prefill_mfma_ok(L)) return fail(MH_E_UNSUPPORTED, "prefill: layer shape not handled by the MFMA path");
     static uint64_t lds_epoch = 0;   // the initialisation the LDS attribute was set under
     if (lds_epoch != init_epoch()) {
-        MH_HIP(hipFuncSetAttribute((const void *)k_moe_gemm<0>, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_lds(2)));
-        MH_HIP(hipFuncSetAttribute((const void *)k_moe_gemm<1>, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_lds(1)));
+        for (const void *f : {(const void *)k_moe_gemm<0, false>, (const void *)k_moe_gemm<0, true>})
+            MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_lds(2)));
+        for (const void *f : {(const void *)k_moe_gemm<1, false>, (const void *)k_moe_gemm<1, true>})
+            MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, gemm_lds(1)));
         lds_epoch = init_epoch();
     }
     unsigned *scale_err_dev = nullptr;
@@ -621,9 +634,12 @@ int run_expert_major_mfma(const DevLayer &L, int n, const float *xb, const int32
         MH_LAUNCH("quant_x", k_quant_terms, dim3((unsigned)((thr + 255) / 256)), dim3(256), 0, s, xb, n, H, qx);
     }
     // gate/up over the quantized tokens, then down over the quantized h
-    MH_LAUNCH("moe_gu_mfma", k_moe_gemm<0>, grid(k_steps(F)), dim3(64 * kWaves), gemm_lds(2), s, A);
+    const bool words = (uintptr_t)L.experts % 16 != 0;
+    auto gu = words ? k_moe_gemm<0, true> : k_moe_gemm<0, false>;
+    auto down = words ? k_moe_gemm<1, true> : k_moe_gemm<1, false>;
+    MH_LAUNCH("moe_gu_mfma", gu, grid(k_steps(F)), dim3(64 * kWaves), gemm_lds(2), s, A);
     A.bq = qh;
-    MH_LAUNCH("moe_down_mfma", k_moe_gemm<1>, grid((H + kRows - 1) / kRows), dim3(64 * kWaves), gemm_lds(1), s, A);
+    MH_LAUNCH("moe_down_mfma", down, grid((H + kRows - 1) / kRows), dim3(64 * kWaves), gemm_lds(1), s, A);
     return hip_check(hipGetLastError(), "prefill MFMA launches");
 }
 

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from conftest import rel_l2, say
-from midge_amd import DevBuf, synth
+from midge_amd import DevBuf, device, synth
 from midge_amd.moe import MoELayer, expert_major_dev
 from midge_amd.synth import Keys, MoEShape
 
@@ -51,3 +51,36 @@ def test_gemm_edges(mh, path_switch, hidden, ffn, plain):
             assert not got[t].any()
         else:
             assert rel_l2(got[t], want[t]) < TOL, (t, sel[t])
+
+
+@pytest.mark.parametrize("hidden,ffn", [(64, 64), (192, 320), (256, 128)])
+@pytest.mark.parametrize("shift", [4, 8, 12])
+def test_table_off_16_bytes(mh, shift, hidden, ffn):
+    """Expert tables on any 4-byte boundary take the matrix cores too, with the
+    same result bit for bit."""
+    say(f"prefill gemm {hidden}x{ffn} table off by {shift}")
+    shape = MoEShape(hidden=hidden, ffn=ffn, n_experts=4, top_k=2)
+    keys = Keys(22)
+    ex = synth.host_layer_experts(shape, keys, 0)
+    w, s, b, nw = synth.host_router(shape, keys, 0)
+    n = 150
+    rng = np.random.default_rng(shift)
+    sel = np.argsort(rng.random((n, 4)), axis=1)[:, :2].astype(np.int32)
+    wt = rng.uniform(0.5, 1.0, (n, 2)).astype(np.float32)
+    xb = rng.standard_normal((n, hidden)).astype(np.float32)
+    out = []
+    for off in (0, shift):
+        table = DevBuf.from_array(np.concatenate([np.zeros(off, np.uint8), ex.view(np.uint8).ravel()]))
+        lay = MoELayer.host(shape, table.ptr + off, w, s, b, nw)
+        bufs = [DevBuf.from_array(a) for a in (xb, sel, wt, np.zeros_like(xb))]
+        device.profile_enable()
+        device.profile_reset()
+        expert_major_dev(lay, n, *bufs)
+        mh.sync()
+        assert device.profile_query("moe_gu_mfma")[1] == 1
+        device.profile_enable(False)
+        out.append(bufs[3].download(np.float32, xb.shape))
+        lay.release()
+        for d in bufs + [table]:
+            d.free()
+    assert np.array_equal(*out) and np.abs(out[0]).max() > 0
