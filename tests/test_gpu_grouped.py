@@ -167,3 +167,101 @@ def test_route(mh, path_switch, kind, n, grouped):
         assert max(rel_l2(a, b) for a, b in zip(*out)) < TOL
     else:
         assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("scales", ["plain", "odd"])
+def test_values_that_are_not_finite(mh, path_switch, scales):
+    """Inputs with infinities, NaN, f32's largest and subnormal numbers: the same
+    infinities and NaN as the GEMVs' f32 sums give, the same bits for the tokens
+    beside them as without them, and subnormal inputs lost without a trace."""
+    shape, n = MID, 24
+    say(f"grouped, values that are not finite, scales={scales}")
+    path_switch("GROUPED")
+    keys, arrays, lay = make(shape, 15, scales)
+    X = synth.host_x(shape, keys, n, step=1)
+    plain = X.copy()
+    X[1, 5] = np.inf
+    X[4, 200] = -np.inf
+    X[7, [0, 255]] = np.inf, -np.inf
+    X[9, 31] = np.nan
+    X[12, 64] = np.nan
+    X[12, 3] = np.inf
+    X[15] *= 1e30          # large, finite sums
+    X[18] *= 1e-42         # subnormal
+    X[20] = 0.0
+    odd = [1, 4, 7, 9, 12, 15, 18, 20]
+    rng = np.random.default_rng(6)
+    sel = rng.integers(0, 6, (n, shape.top_k)).astype(np.int32)   # groups that odd and plain tokens share
+    w = rng.uniform(0.5, 1.0, (n, shape.top_k)).astype(np.float32)
+    out = []
+    for x, gemv in ((X, False), (X, True), (plain, False)):
+        path_switch("NO_MFMA", gemv)
+        bufs = [DevBuf.from_array(a) for a in (x, sel, w, np.zeros_like(X))]
+        expert_major_dev(lay, n, *bufs)
+        mh.sync()
+        out.append(bufs[3].download(np.float32, X.shape))
+        for d in bufs:
+            d.free()
+    lay.release()
+    got, want, alone = out
+    assert not np.isfinite(want[[1, 4, 7, 9, 12]]).all()
+    assert (np.isnan(got) == np.isnan(want)).all() and (np.isposinf(got) == np.isposinf(want)).all()
+    assert (np.isneginf(got) == np.isneginf(want)).all()
+    rest = np.setdiff1d(np.arange(n), odd)
+    assert np.array_equal(got[rest], alone[rest])
+    for t in list(rest) + [15, 18, 20]:
+        assert np.isfinite(want[t]).all() and rel_l2(got[t], want[t]) < TOL, t
+
+
+def experts_f64(shape, ex, xb, sel, w):
+    """sum_i w_i expert_{sel_i}(xb) per token in 64 bits, from the layer's bytes."""
+    lay, out = shape.layout, np.zeros(xb.shape)
+    code = np.array([0, 0.5, 1, 1.5, 2, 3, 4, 6, 0, -0.5, -1, -1.5, -2, -3, -4, -6])
+
+    def matrix(e, m):
+        rows, cols = lay.rows[m], lay.cols[m]
+        q = ex[lay.offset(0, e, m, 0):][:rows * cols // 2].reshape(rows, -1)
+        sc = ex[lay.offset(0, e, m, 1):][:rows * cols // 16].view(np.float16).astype(np.float64).reshape(rows, -1)
+        b = ex[lay.offset(0, e, m, 2):][:4 * rows].view(np.float32).astype(np.float64)
+        v = np.stack((code[q & 15], code[q >> 4]), -1).reshape(rows, cols // 32, 32)
+        return (v * sc[:, :, None]).reshape(rows, cols), b
+
+    for e in np.unique(sel):
+        t, i = np.nonzero(sel == e)
+        (wg, bg), (wu, bu), (wd, bd) = (matrix(e, m) for m in range(3))
+        x = xb[t].astype(np.float64)
+        g, u = np.minimum(x @ wg.T + bg, shape.limit), np.clip(x @ wu.T + bu, -shape.limit, shape.limit)
+        h = g / (1 + np.exp(-shape.alpha * g)) * (u + 1)
+        np.add.at(out, t, (h @ wd.T + bd) * w[t, i, None].astype(np.float64))
+    return out
+
+
+@pytest.mark.parametrize("hidden,ffn", [(256, 192), (512, 2048), (1024, 768), (2880, 2880)])
+def test_error_against_64_bits(mh, path_switch, hidden, ffn):
+    """The grouped kernels hold an input to 23 bits (two f16 terms) where the
+    GEMVs have f32's 24, and add in longer chains of the matrix core where those
+    add lane by lane: their outputs are no further from 64 bits."""
+    shape = MoEShape(hidden=hidden, ffn=ffn, n_experts=4, top_k=2)
+    say(f"grouped error {hidden}x{ffn}")
+    path_switch("GROUPED")
+    keys, (ex, *_), lay = make(shape, 16)
+    n = 15   # fewer than 8 assignments per expert
+    rng = np.random.default_rng(hidden)
+    err = []
+    for rep in range(4):
+        xb = rng.standard_normal((n, hidden)).astype(np.float32)
+        sel = np.argsort(rng.random((n, 4)), axis=1)[:, :2].astype(np.int32)
+        w = rng.uniform(0.2, 0.8, (n, 2)).astype(np.float32)
+        want = experts_f64(shape, ex.view(np.uint8).ravel(), xb, sel, w)
+        for gemv in (False, True):
+            path_switch("NO_MFMA", gemv)
+            bufs = [DevBuf.from_array(a) for a in (xb, sel, w, np.zeros_like(xb))]
+            expert_major_dev(lay, n, *bufs)
+            mh.sync()
+            err.append(rel_l2(bufs[3].download(np.float32, xb.shape), want))
+            for d in bufs:
+                d.free()
+    lay.release()
+    grouped, gemv = np.sqrt(np.mean(np.square(err[0::2]))), np.sqrt(np.mean(np.square(err[1::2])))
+    say(f"grouped {grouped:.3g}, GEMVs {gemv:.3g}")
+    assert grouped < 1.02 * gemv < 4e-7
