@@ -867,7 +867,7 @@ def prefill_probe(ev, s, seed: int, n: int = 512, reps: int = 10) -> dict:
                 expert_major_dev(lay, n, xb, sel, w, x)
                 midge_amd.sync()
                 kern = {}
-                for name in ("plist", "quant_x", "moe_gu_mfma", "quant_h", "moe_down_mfma", "combine_prefill"):
+                for name in ("plist", "quant_x", "moe_gu_mfma", "moe_down_mfma", "combine_prefill"):
                     tot, cnt = profile_query(name)
                     if cnt:
                         kern[name] = {"us": 1e3 * tot, "launches": cnt}

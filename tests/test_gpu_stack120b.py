@@ -125,6 +125,9 @@ def test_stack_decode_vs_oracle(stack, batch, check, calls):
             d.free()
         for l in range(nl):
             assert (usage[l] == np.bincount(sel[l].ravel(), minlength=SHAPE.n_experts)).all()
+        assert np.isfinite(got).all()
+        if not with_ref:   # (a chain's bar is twice the reference's own divergence from the oracle over it)
+            pytest.skip("reference engine not built (oracle/_ref): it sets the chains' bar")
         for t in check:
             say(f"oracle chain token {t} of batch {batch} call {call}")
             xr, xa, tie = oracle_chain(keys, X[t].copy(), sel[:, t], with_ref)
