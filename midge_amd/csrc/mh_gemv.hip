@@ -656,7 +656,12 @@ int launch_gemm_q8r(const DevWT &w, const float *x, float *y, int batch, hipStre
         (uintptr_t)w.data % 16 != 0)
         return MH_OK;
     if (sw(SW_NO_MFMA)) return MH_OK;
-    // the long tiling when it gives every SIMD two waves, else the K-split one
+    // Long matrices: where the register-operand kernel's long tiling gives every
+    // SIMD two waves (131072 rows on 256 CUs), which is where it overtakes its
+    // K-split tiling. The LDS kernel took over that line with the matrices; its
+    // own lies lower (2880 columns at batch 2 / 64, LDS against K-split: 5120
+    // rows 18 / 34 us against 11 / 25, 16384 20 / 35 against 23 / 69, 65536 33 / 52
+    // against 79 / 270).
     const bool longm = (R + Q8Long::rows - 1) / Q8Long::rows * (Q8Long::threads / 64) >= 2 * 4 * device_cus();
     const bool rows = longm && !sw(SW_Q8_NO_ROWS);
     // groups of up to 64 columns (the row kernel) or 32, as even as 16-column tiles allow

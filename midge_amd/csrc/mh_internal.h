@@ -157,7 +157,7 @@ int step_plan_create(const DevLayer *layers, int n_layers, StepPlan **out);
 void step_plan_destroy(StepPlan *p);
 bool step_plan_ok(const StepPlan *p);
 // 1 if every MXFP4 scale of the plan's layers is f16-exact (the expert-
-// grouped matrix-core kernels may run them).
+// grouped matrix-core kernels then run without a look at the scales).
 bool step_plan_few(const StepPlan *p);
 // A layer's assignments by expert: order[r] = assignment a of sorted position
 // r, order[N + r] = its expert (unroutable ones last, -1), and the same in

@@ -559,8 +559,10 @@ int launch_expert_lists(const int32_t *sel, int N, int E, int k, ExpertLists *ou
     return hip_check(hipGetLastError(), "expert lists launch");
 }
 
-// The widest layers that the scaled-MFMA path takes (wider ones keep the
-// per-assignment GEMVs' f32 arithmetic).
+// The widest layers that the scaled-MFMA path takes. The kernel itself has no
+// need of a bound; layers past it have always had the per-assignment GEMVs' f32
+// arithmetic, and keep it (the fp6 terms hold an activation to 2^-12 of its
+// block's largest).
 constexpr int64_t kMfmaMaxH = 3328, kMfmaMaxF = 4608;
 
 // True when the scaled-MFMA path handles this layer (MXFP4 experts on a 4-byte
