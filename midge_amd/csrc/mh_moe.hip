@@ -1104,11 +1104,14 @@ bool decode_grouped(const DevLayer &L, int n, bool exact) {
     return sw(SW_GROUPED) || (exact && n <= 16 && n * L.top_k <= 64) || grouped_pays(L, n);
 }
 // Whether the router writes a table: for the grouped kernels, and up to 16
-// tokens, where the top-k's own block does it, for the GEMVs of layers that those
-// cannot run, to walk the assignments by expert (with few assignments it gains
-// less than the 1.2 us that it takes).
+// tokens, where the top-k's own block does it, for the GEMVs to walk the
+// assignments by expert, in layers that the grouped kernels cannot run and
+// where the assignments' weights are past 200 MB (it takes 1.2 us; 4 tokens,
+// top-8 of 64 experts, 2880 wide 104 us with it, 108 without; 2 tokens, top-2 of
+// 32, 1024 x 768 32.3 and 31.0).
 bool decode_table(const DevLayer &L, int n, bool exact) {
-    return decode_grouped(L, n, exact) || (n <= 16 && !grouped_ok(L, n));
+    return decode_grouped(L, n, exact) ||
+           (n <= 16 && (!grouped_ok(L, n) || (double)n * L.top_k * (double)L.expert_stride > 200e6));
 }
 
 // exact: the layer's scales are known to be carried by f16 (a stack's plan
